@@ -89,6 +89,8 @@ def draw(rng):
     if op in ("linear", "pre"):
         M = 1 if rng.random() < 0.45 else rng.choice((2, 3, 4, 5, 6, 7, 8, 10, 12, 16, 16))
         K = _k(rng)
+        while M > 1 and K % (2 * va.GROUP[qtype]) and M * K > 55000:  # an odd number of groups: rows that fit a workgroup
+            M //= 2
         N = _log(rng, 512, 28672)
         if rng.random() < 0.5:
             N = max(512, N // 256 * 256)
