@@ -21,8 +21,6 @@ namespace vq {
 //                every workgroup recomputes the row's sum of squares);
 //   PRO_SWIGLU   bf16 gate and up: v = bf16(silu(g) * u) (silu_mul), then
 //                quantized (swiglu_quantize.cu:35-78 folded in).
-// The two folded prologues need the whole row in one load round
-// (K / 8 <= M1_XS * NTT octets).
 //
 // Up to three matrices with the same K may share a launch (q/k/v, gate/up):
 // workgroups [0, e0) work on matrix 0, [e0, e1) on matrix 1, the rest on
@@ -38,8 +36,7 @@ namespace vq {
 // {-OFF * sum(q) over the chunk (int32), xs (fp32)}, 16 floats of cross-wave
 // sums and, for exact tilings, the workgroup's block of weight scales.
 
-constexpr int M1_XS = 4;    // activation octets per thread loaded before the weights
-constexpr int M1_XS_MR = 8; // the same for MR > 1 rows (all of them: no later rounds)
+constexpr int M1_XS_MR = 8; // MR > 1 rows: most activation octets per thread (all loaded before the weights)
 constexpr int M1_DELAY = 6; // weight-issue delay, s_sleep units (one activation row)
 constexpr int M1_DELAY_MR = 8; // the same for MR > 1 bf16 rows (MR rows of activation ahead of the weights)
 constexpr int M1_DELAY_ROUND = 4; // the same for MR > 1 int8 rows, per staging round of the rows
@@ -271,6 +268,63 @@ __device__ __forceinline__ uint16_t* m1_xout() {
     return *(uint16_t* const __attribute__((address_space(4)))*)(ka + offsetof(M1KernArgs, xout) + z);
 }
 
+// PRO_RMSNORM / PRO_SWIGLU: one octet of the bf16 row element-wise from two inputs
+template <int PRO>
+__device__ __forceinline__ u32x4 m1_produce(const u32x4& v, const u32x4& a, float inv) {
+    const uint32_t vw[4] = {v.x, v.y, v.z, v.w}, aw[4] = {a.x, a.y, a.z, a.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float f0 = bf16f(vw[j] & 0xffffu), f1 = bf16f(vw[j] >> 16);
+        const float g0 = bf16f(aw[j] & 0xffffu), g1 = bf16f(aw[j] >> 16);
+        if constexpr (PRO == PRO_RMSNORM) {
+            f0 = (f0 * inv) * g0;
+            f1 = (f1 * inv) * g1;
+        } else {
+            f0 = silu_mul(f0, g0);
+            f1 = silu_mul(f1, g1);
+        }
+        o[j] = f2bf2(f0, f1);
+    }
+    return u32x4{o[0], o[1], o[2], o[3]};
+}
+
+// Stage octet o (of noct) into the LDS row: the bf16 octet quantized, or (PRE)
+// {int8 octet, int8 octet, group scale of a chunk's first octet} rearranged.
+// Q4 stores each octet as (ql nibbles, qh nibbles); Q5/Q6 as [k even | k odd]
+// int8; W8 in k order.  All lanes of the octet's group call this together.
+template <int F, bool PRE>
+__device__ __forceinline__ void m1_quant_store(int o, const u32x4& v, int noct, int8_t* lxq, u32x2* lcs) {
+    using FT = Fmt<F>;
+    constexpr int OPC = FT::CK / 8;  // octets per chunk
+    uint32_t d0, d1;
+    float s;
+    if constexpr (PRE) {
+        d0 = v.x;
+        d1 = v.y;
+        if constexpr (F == 5 || F == 6) {
+            d0 = __builtin_amdgcn_perm(v.y, v.x, 0x06040200u);
+            d1 = __builtin_amdgcn_perm(v.y, v.x, 0x07050301u);
+        }
+        s = __uint_as_float(v.z);
+    } else {
+        quantize_octet<FT::G, (F == 5 || F == 6)>(v, d0, d1, s);
+    }
+    int corr = 0;
+    if constexpr (F == 4) {
+        const uint32_t ql = nibbles8(d0, d1), qh = nibbles8(d0 >> 4, d1 >> 4);
+        d0 = ql;
+        d1 = qh;
+        corr = -8 * group_sum<OPC>((int)udot8(ql, 0x11111111u, 0u));
+    } else if constexpr (FT::OFF != 0) {
+        corr = -FT::OFF * group_sum<OPC>(bytesum8(d0, d1));
+    }
+    if (o < noct) {
+        *(u32x2*)(lxq + (size_t)o * 8) = u32x2{d0, d1};
+        if (o % OPC == 0) lcs[o / OPC] = u32x2{(uint32_t)corr, __float_as_uint(s)};
+    }
+}
+
 // EXACT: every lane's chunks lie inside its row (the row has exactly TS * CPL
 // chunks) and a row's scales fill whole 16-byte words (groups % 8 == 0), so no
 // chunk needs masking and the workgroup's scale block is loaded with one
@@ -293,7 +347,7 @@ __device__ __forceinline__ uint16_t* m1_xout() {
 // (x [M][K], y and the residual [M][N]); every workgroup stages all M rows,
 // each lane decodes its weight chunk once and dots it with every row.  Small
 // verify batches then need no separate quantize launch.
-template <int F, int TS, int NTT, int CPL, int SENC, int MODE, bool EXACT, int PRO, int MR, int DELAY, int KC = 0>
+template <int F, int TS, int NTT, int CPL, int SENC, int MODE, bool EXACT, int PRO, int MR, int DELAY>
 __global__ void __launch_bounds__(NTT)
 qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* y0, int K, int n0, int e0,
                 int e1, const uint16_t* res, const void* xa, float eps, uint16_t* __restrict__ xout,
@@ -316,13 +370,8 @@ qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* 
     // exact tilings: K is the tiling's row length and the argument slot
     // carries the grid size instead (for the XCD-aware block order); the
     // load rounds of one row are then exact
-    // KC (masked exact tilings): the row has KC < TS * CPL chunks; K is still
-    // the constant, the scale block still staged, and the slots past the row
-    // read nothing (out of the buffer's range) and add nothing.
-    constexpr int KX = EXACT ? (KC ? Fmt<F>::CK * KC : m1_exact_k<F>(TS, CPL)) : 0;
-    constexpr bool MASK = EXACT && KC != 0 && KC != TS * CPL;
-    static_assert(!MASK || (MR == 1 && KC < TS * CPL), "masked tilings: one row, fewer chunks than slots");
-    constexpr bool FULL = EXACT && !MASK;  // every slot holds a chunk of the row
+    constexpr int KX = EXACT ? m1_exact_k<F>(TS, CPL) : 0;
+    static_assert(EXACT || MR > 1, "one row: exact tilings");
     const int grid = K;
     if constexpr (EXACT) K = KX;
     // SPARE: the first wave stages no activation and issues its weights at
@@ -367,7 +416,7 @@ qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* 
     // against 2.64 us).
     constexpr bool PAIR8 = PRE && !SPARE && m1_pairs<F>(EXACT, NTT, MR, PRO);
     constexpr int XS = (PAIR8 || PAIRBF) ? (MR * (KX / 16) + ANT - 1) / ANT
-                       : EXACT ? (MR * (KX / 8) + ANT - 1) / ANT : MR > 1 ? M1_XS_MR : M1_XS;
+                       : EXACT ? (MR * (KX / 8) + ANT - 1) / ANT : M1_XS_MR;
     constexpr int ROWS = NTT / TS;
     const int M = MR == 1 ? 1 : e1;  // activation rows
     constexpr int HB = FT::HIW * 4;  // high-plane bytes per chunk: Q5 4, Q6 8
@@ -445,16 +494,6 @@ qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* 
     constexpr int OPG = FT::G / 8;   // octets per group
     const auto xr = buf(x, (uint32_t)(M * K) * (PRE ? 1 : 2));
     const auto xsr = buf(xa, PRE ? (uint32_t)(M * (K / FT::G)) * 4 : TWO ? (uint32_t)K * 2 : 0u);
-    // bf16 octet, or {int8 octet, int8 octet, group scale of a chunk's first octet}
-    auto load_x = [&](int o) -> u32x4 {
-        if constexpr (PRE) {
-            const u32x2 q = bload8(xr, o * 8);
-            const uint32_t sb = bload4(xsr, (o % OPC == 0) ? (o / OPG) * 4 : OOB);
-            return u32x4{q.x, q.y, sb, 0u};
-        } else {
-            return bload16(xr, o * 16);
-        }
-    };
     // rounds past the row are not issued (the bound is workgroup-uniform)
     // The first input's octets go out first: the second input (int8 group
     // scales, gamma, up) sits past the 14 preloaded argument dwords, and the
@@ -527,7 +566,7 @@ qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* 
 #pragma unroll
         for (int j = 0; j < CPL; ++j) {
             const int c = seg * segw + j * TS + l;
-            const bool in = FULL || c < CPR;
+            const bool in = EXACT || c < CPR;
             wv[j] = bload16<AUX_NT>(wr, in ? rt * (int)rbytes + c * 16 : OOB);
             // odd lanes and chunks past the row read scale 0, which zeroes
             // their term without any select
@@ -580,53 +619,8 @@ qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* 
         for (int i = 0; i < NTT / 64; ++i) t += lred[i];
         inv = __builtin_amdgcn_rsqf(t / (float)K + epsv);
     }
-    // PRO_RMSNORM / PRO_SWIGLU: the bf16 row element-wise from two inputs
-    auto produce = [&](const u32x4& v, const u32x4& a) -> u32x4 {
-        const uint32_t vw[4] = {v.x, v.y, v.z, v.w}, aw[4] = {a.x, a.y, a.z, a.w};
-        uint32_t o[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float f0 = bf16f(vw[j] & 0xffffu), f1 = bf16f(vw[j] >> 16);
-            const float g0 = bf16f(aw[j] & 0xffffu), g1 = bf16f(aw[j] >> 16);
-            if constexpr (PRO == PRO_RMSNORM) {
-                f0 = (f0 * inv) * g0;
-                f1 = (f1 * inv) * g1;
-            } else {
-                f0 = silu_mul(f0, g0);
-                f1 = silu_mul(f1, g1);
-            }
-            o[j] = f2bf2(f0, f1);
-        }
-        return u32x4{o[0], o[1], o[2], o[3]};
-    };
-    auto quant_store = [&](int o, const u32x4& v) {
-        uint32_t d0, d1;
-        float s;
-        if constexpr (PRE) {
-            d0 = v.x;
-            d1 = v.y;
-            if constexpr (F == 5 || F == 6) {
-                d0 = __builtin_amdgcn_perm(v.y, v.x, 0x06040200u);
-                d1 = __builtin_amdgcn_perm(v.y, v.x, 0x07050301u);
-            }
-            s = __uint_as_float(v.z);
-        } else {
-            quantize_octet<FT::G, (F == 5 || F == 6)>(v, d0, d1, s);
-        }
-        int corr = 0;
-        if constexpr (F == 4) {
-            const uint32_t ql = nibbles8(d0, d1), qh = nibbles8(d0 >> 4, d1 >> 4);
-            d0 = ql;
-            d1 = qh;
-            corr = -8 * group_sum<OPC>((int)udot8(ql, 0x11111111u, 0u));
-        } else if constexpr (FT::OFF != 0) {
-            corr = -FT::OFF * group_sum<OPC>(bytesum8(d0, d1));
-        }
-        if (o < noct) {
-            *(u32x2*)(lxq + (size_t)o * 8) = u32x2{d0, d1};
-            if (o % OPC == 0) lcs[o / OPC] = u32x2{(uint32_t)corr, __float_as_uint(s)};
-        }
-    };
+    auto produce = [&](const u32x4& v, const u32x4& a) { return m1_produce<PRO>(v, a, inv); };
+    auto quant_store = [&](int o, const u32x4& v) { m1_quant_store<F, PRE>(o, v, noct, lxq, lcs); };
     const int wave0 = (tid & ~63) - A0;  // waves with no octet skip the quantize
 #pragma unroll
     for (int i = 0; i < XS; ++i) {
@@ -677,11 +671,6 @@ qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* 
             }
         }
     }
-    if constexpr (!TWO && MR == 1 && !PAIR8 && !PAIRBF) {
-        if (__builtin_expect(xiters > XS, 0))
-            for (int i = XS; i < xiters; ++i)
-                if (stager && wave0 + ANT * i < noct) quant_store(at + ANT * i, load_x(at + ANT * i));
-    }
 
     // the scale block into LDS after the activation: its loads come from HBM
     // and arrive after the activation's, and the quantize (and the rmsnorm
@@ -703,47 +692,32 @@ qgemv_m1_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16_t* 
         return;
     }
     float acc = 0.0f;
-    for (int seg = 0; seg < nseg; ++seg) {
-        if (seg) load_seg(seg);
-        u32x4 A0[CPL], A1[CPL];
-        u32x2 CS[CPL];
-        float SC[CPL];  // ws * xs of the chunk's group (0 on the odd lane of a pair)
+    u32x4 X0[CPL], X1[CPL];
+    u32x2 CS[CPL];
+    float SC[CPL];  // ws * xs of the chunk's group (0 on the odd lane of a pair)
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-            const int c = seg * segw + j * TS + l;
-            const int cc = FULL ? c : min(c, CPR - 1);
-            CS[j] = lcs[cc];
-            const u32x4* a = (const u32x4*)(lxq + (size_t)cc * FT::CK);
-            A0[j] = a[0];
-            A1[j] = FT::OFF ? a[1] : a[0];
-            if constexpr (EXACT) {
-                // read on every lane (in bounds), select after: no branch, no
-                // wait between the LDS reads, product formed before the weights
-                // (a masked slot's scale is 0: its dot of zero weights with the
-                // last chunk's activation adds nothing)
-                const uint32_t sraw = lsc[rr * NGR + (cc >> 1)];
-                const float wsf = SENC ? bf16f(sraw) : f16f(sraw);
-                SC[j] = ((lead && (FULL || c < CPR)) ? wsf : 0.0f) * __uint_as_float(CS[j].y);
-            }
-        }
+    for (int j = 0; j < CPL; ++j) {
+        const int c = j * TS + l;
+        CS[j] = lcs[c];
+        const u32x4* a = (const u32x4*)(lxq + (size_t)c * FT::CK);
+        X0[j] = a[0];
+        X1[j] = FT::OFF ? a[1] : a[0];
+        // read on every lane (in bounds), select after: no branch, no wait
+        // between the LDS reads, product formed before the weights
+        const uint32_t sraw = lsc[rr * NGR + (c >> 1)];
+        const float wsf = SENC ? bf16f(sraw) : f16f(sraw);
+        SC[j] = (lead ? wsf : 0.0f) * __uint_as_float(CS[j].y);
+    }
 #pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-            const int c = seg * segw + j * TS + l;
-            const bool ok = FULL || c < CPR;
-            const int cc = FULL ? c : min(c, CPR - 1);
-            int dot;
-            if constexpr (F == 4) dot = chunk_dot_q4(wv[j], A0[j], A1[j], (int)CS[j].x);
-            else dot = chunk_dot<F>(wv[j], h0[j], h1[j], A0[j], A1[j], (int)CS[j].x);
-            dot += dpp_i<DPP_SWAP1>(dot);
-            const int g = cc >> 1;
-            if constexpr (PART)
-                if (ok && lead && row_ok) part[(size_t)row * NGR + g] = dot;
-            float scj;
-            if constexpr (EXACT) scj = SC[j];
-            else scj = (SENC ? bf16f(sv[j]) : f16f(sv[j])) * __uint_as_float(CS[j].y);
-            acc = __builtin_fmaf(scj, (float)dot, acc);
-            if (j == 0) stamp(5);
-        }
+    for (int j = 0; j < CPL; ++j) {
+        int dot;
+        if constexpr (F == 4) dot = chunk_dot_q4(wv[j], X0[j], X1[j], (int)CS[j].x);
+        else dot = chunk_dot<F>(wv[j], h0[j], h1[j], X0[j], X1[j], (int)CS[j].x);
+        dot += dpp_i<DPP_SWAP1>(dot);
+        if constexpr (PART)
+            if (lead && row_ok) part[(size_t)row * NGR + ((j * TS + l) >> 1)] = dot;
+        acc = __builtin_fmaf(SC[j], (float)dot, acc);
+        if (j == 0) stamp(5);
     }
     stamp(6);
     acc = team_sum<TS>(acc);
@@ -781,87 +755,75 @@ typedef void (*m1_fn)(const void*, const uint8_t*, const uint16_t*, uint16_t*, i
                       const void*, float, uint16_t*, int32_t*, const uint8_t*, const uint16_t*, uint16_t*, int,
                       const uint8_t*, const uint16_t*, uint16_t*, int);
 
-// Launch shapes instantiated for every format: (team size, workgroup size,
-// chunk slots per lane).
-// 5 slots tile K = 2560 (Q4/Q5/Q6: 16 lanes), 5120 and 10240; 6 slots tile
-// the reference engine's K = 3072 (16 lanes; W8: 32), 6144 (32; W8: 64) and
-// 12288 (64 lanes).
-// The 384-thread ones spread the engine's q (N = 6144) and o (N = 3072) over
-// exactly one workgroup per CU (24 / 12 rows), where 256 / 320 threads left
-// some CUs with twice the rows of others.
+// Launch shapes: (team size, workgroup size, chunk slots per lane).  One row:
+// the exact tilings of 80 and 96 chunks (K = 2560 and the reference engine's
+// 3072; the 384-thread one puts the engine's shorter matrices on exactly one
+// workgroup per CU), for W8 also 160 and 192 (the same K); every other K takes
+// the streaming kernel (qgemv_stream.h).  The longer ones serve 2-4 rows.
 constexpr int M1_SHAPES[][3] = {{8, 128, 10}, {8, 192, 10}, {8, 320, 10}, {16, 256, 10}, {16, 640, 10},
-                                {32, 320, 10}, {32, 640, 10}, {64, 640, 10}, {16, 256, 5}, {16, 320, 5},
-                                {16, 640, 5}, {32, 640, 5}, {64, 640, 5}, {16, 256, 6}, {16, 320, 6},
-                                {16, 384, 6}, {32, 320, 6}, {32, 384, 6}, {32, 640, 6}, {64, 640, 6}};
-// Masked exact tilings (team size, workgroup size, chunk slots per lane,
-// chunks per row): rows with no exact tiling of at most 10 slots per lane
-// keep K constant and the staged scale block, and mask the last slots.  336
-// chunks: the engine's K = 10752 (Q4/Q5/Q6), 64 lanes x 6 slots; 384 and 768
-// threads put the engine's N = 3072 on 512 / 256 workgroups (6 / 12 rows).
+                                {32, 640, 10}, {64, 640, 10}, {16, 256, 5}, {16, 320, 5}, {16, 640, 5},
+                                {32, 640, 5}, {64, 640, 5}, {16, 256, 6}, {16, 320, 6}, {16, 384, 6},
+                                {32, 320, 6}, {32, 384, 6}, {32, 640, 6}};
 // One Q4 / Q5 matrix of 96 chunks per row (K = 3072) whose 384-thread
 // workgroups leave the CUs unevenly loaded: an 11-wave workgroup of 44 rows
 // (m1_wide96 says when).
 constexpr int M1_WIDE96[3] = {16, 704, 6};
-constexpr int M1_MASKED[][4] = {{64, 320, 6, 336}, {64, 384, 6, 336}, {64, 640, 6, 336}, {64, 768, 6, 336}};
 
-// Shapes of 5 or 6 chunk slots per lane are only ever exact tilings (m1_shape
-// picks those by TS * CPL == chunks per row, or a masked tiling's chunks per
-// row; other rows take 10 slots), so their non-exact variants are not built.
+// Rows of `cpr` chunks that one-row launches tile exactly here.  (At 160 and
+// more chunks of the nibble formats the streaming kernel is faster: K = 5120,
+// N = 4096 / 11008 4.19 / 7.64 -> 3.95 / 6.95 us, K = 10240, N = 2560 / 11008
+// 4.52 / 14.4 -> 4.37 / 11.6 us; at 80 and 96 it is equal or slower: K = 2560,
+// N = 2560 / 10240 2.70 / 4.5 against 2.83 / 4.5 us.)
+__host__ __device__ constexpr bool m1_tiles(int f, int cpr) {
+    return cpr == 80 || cpr == 96 || (f == 8 && (cpr == 160 || cpr == 192));
+}
+
 template <int F, int SENC, int MODE, bool EXACT, int PRO, int MR>
-m1_fn m1_kernel_v(int ts, int ntt, int cpl, int kc) {
+m1_fn m1_kernel_v(int ts, int ntt, int cpl) {
 #define VQ_M1(TS_, NTT_, CPL_)                                                                      \
     if constexpr ((EXACT || CPL_ == 10) && (MODE != M1_SWIGLU || m1_pair_ok(TS_, NTT_)) &&          \
-                  (MR == 1 || m1_mr_shape_ok(TS_, NTT_, CPL_)))                                     \
-        if (ts == TS_ && ntt == NTT_ && cpl == CPL_ && kc == 0)                                     \
+                  (MR == 1 ? EXACT && m1_tiles(F, TS_ * CPL_) : m1_mr_shape_ok(TS_, NTT_, CPL_)))    \
+        if (ts == TS_ && ntt == NTT_ && cpl == CPL_)                                                \
             return qgemv_m1_kernel<F, TS_, NTT_, CPL_, SENC, MODE, EXACT, PRO, MR,                          \
                                    m1_delay<F>(EXACT, TS_, NTT_, CPL_, MODE, MR, PRO)>;
     VQ_M1(8, 128, 10) VQ_M1(8, 192, 10) VQ_M1(8, 320, 10) VQ_M1(16, 256, 10) VQ_M1(16, 640, 10)
-    VQ_M1(32, 320, 10) VQ_M1(32, 640, 10) VQ_M1(64, 640, 10) VQ_M1(16, 256, 5) VQ_M1(16, 320, 5)
-    VQ_M1(16, 640, 5) VQ_M1(32, 640, 5) VQ_M1(64, 640, 5) VQ_M1(16, 256, 6) VQ_M1(16, 320, 6)
-    VQ_M1(16, 384, 6) VQ_M1(32, 320, 6) VQ_M1(32, 384, 6) VQ_M1(32, 640, 6) VQ_M1(64, 640, 6)
+    VQ_M1(32, 640, 10) VQ_M1(64, 640, 10) VQ_M1(16, 256, 5) VQ_M1(16, 320, 5) VQ_M1(16, 640, 5)
+    VQ_M1(32, 640, 5) VQ_M1(64, 640, 5) VQ_M1(16, 256, 6) VQ_M1(16, 320, 6) VQ_M1(16, 384, 6)
+    VQ_M1(32, 320, 6) VQ_M1(32, 384, 6) VQ_M1(32, 640, 6)
     // the 44-row workgroup of one Q4 / Q5 matrix at K = 3072 (M1_WIDE96), bf16 or int8 row
     if constexpr (F == 4 || F == 5)
         if constexpr (MR == 1 && MODE != M1_SWIGLU && (PRO == PRO_BF16 || PRO == PRO_INT8))
             VQ_M1(M1_WIDE96[0], M1_WIDE96[1], M1_WIDE96[2])
 #undef VQ_M1
-    // masked exact tilings (KC_ chunks in TS_ * CPL_ slots), one row
-#define VQ_M1K(TS_, NTT_, CPL_, KC_)                                                                \
-    if constexpr (EXACT && MR == 1 && (MODE != M1_SWIGLU || m1_pair_ok(TS_, NTT_)))                  \
-        if (ts == TS_ && ntt == NTT_ && cpl == CPL_ && kc == KC_)                                   \
-            return qgemv_m1_kernel<F, TS_, NTT_, CPL_, SENC, MODE, EXACT, PRO, MR,                          \
-                                   m1_delay<F>(EXACT, TS_, NTT_, CPL_, MODE, MR, PRO), KC_>;
-    VQ_M1K(64, 320, 6, 336) VQ_M1K(64, 384, 6, 336) VQ_M1K(64, 640, 6, 336) VQ_M1K(64, 768, 6, 336)
-#undef VQ_M1K
     return nullptr;
 }
 
 template <int F, int PRO, int MODE, int MR>
-m1_fn m1_pick_mode(int ts, int ntt, int cpl, int kc, int senc, bool exact) {
+m1_fn m1_pick_mode(int ts, int ntt, int cpl, int senc, bool exact) {
     if (exact)
-        return senc ? m1_kernel_v<F, 1, MODE, true, PRO, MR>(ts, ntt, cpl, kc)
-                    : m1_kernel_v<F, 0, MODE, true, PRO, MR>(ts, ntt, cpl, kc);
-    if (kc != 0) return nullptr;
-    return senc ? m1_kernel_v<F, 1, MODE, false, PRO, MR>(ts, ntt, cpl, 0)
-                : m1_kernel_v<F, 0, MODE, false, PRO, MR>(ts, ntt, cpl, 0);
+        return senc ? m1_kernel_v<F, 1, MODE, true, PRO, MR>(ts, ntt, cpl)
+                    : m1_kernel_v<F, 0, MODE, true, PRO, MR>(ts, ntt, cpl);
+    return senc ? m1_kernel_v<F, 1, MODE, false, PRO, MR>(ts, ntt, cpl)
+                : m1_kernel_v<F, 0, MODE, false, PRO, MR>(ts, ntt, cpl);
 }
 // The swiglu pair is built for the BF16 and RMSNORM prologues (the inputs of
 // the engine's gate/up projection); MR > 1 rows for BF16 and INT8; the
 // partials (test entry point viper_hip_qlinear_partials) for BF16 only, the
 // one prologue that entry point takes.
 template <int F, int PRO>
-m1_fn m1_pick_pro(int ts, int ntt, int cpl, int kc, int senc, int mode, bool exact, int mr) {
+m1_fn m1_pick_pro(int ts, int ntt, int cpl, int senc, int mode, bool exact, int mr) {
     constexpr bool PART_OK = PRO == PRO_BF16;
     if constexpr (PRO == PRO_BF16 || PRO == PRO_INT8) {
         if (mr == 2) {
             if constexpr (PART_OK)
-                if (mode == M1_PART) return m1_pick_mode<F, PRO, M1_PART, 2>(ts, ntt, cpl, kc, senc, exact);
-            if (mode == M1_PLAIN) return m1_pick_mode<F, PRO, M1_PLAIN, 2>(ts, ntt, cpl, kc, senc, exact);
+                if (mode == M1_PART) return m1_pick_mode<F, PRO, M1_PART, 2>(ts, ntt, cpl, senc, exact);
+            if (mode == M1_PLAIN) return m1_pick_mode<F, PRO, M1_PLAIN, 2>(ts, ntt, cpl, senc, exact);
             return nullptr;
         }
         if (mr == 4) {
             if constexpr (PART_OK)
-                if (mode == M1_PART) return m1_pick_mode<F, PRO, M1_PART, 4>(ts, ntt, cpl, kc, senc, exact);
-            if (mode == M1_PLAIN) return m1_pick_mode<F, PRO, M1_PLAIN, 4>(ts, ntt, cpl, kc, senc, exact);
+                if (mode == M1_PART) return m1_pick_mode<F, PRO, M1_PART, 4>(ts, ntt, cpl, senc, exact);
+            if (mode == M1_PLAIN) return m1_pick_mode<F, PRO, M1_PLAIN, 4>(ts, ntt, cpl, senc, exact);
             return nullptr;
         }
     }
@@ -870,34 +832,34 @@ m1_fn m1_pick_pro(int ts, int ntt, int cpl, int kc, int senc, int mode, bool exa
     if constexpr (PRO == PRO_BF16)
         if (mode == M1_TL)
             return !exact ? nullptr
-                          : senc ? m1_kernel_v<F, 1, M1_TL, true, PRO, 1>(ts, ntt, cpl, kc)
-                                 : m1_kernel_v<F, 0, M1_TL, true, PRO, 1>(ts, ntt, cpl, kc);
+                          : senc ? m1_kernel_v<F, 1, M1_TL, true, PRO, 1>(ts, ntt, cpl)
+                                 : m1_kernel_v<F, 0, M1_TL, true, PRO, 1>(ts, ntt, cpl);
     if constexpr (PART_OK)
-        if (mode == M1_PART) return m1_pick_mode<F, PRO, M1_PART, 1>(ts, ntt, cpl, kc, senc, exact);
+        if (mode == M1_PART) return m1_pick_mode<F, PRO, M1_PART, 1>(ts, ntt, cpl, senc, exact);
     if constexpr (PRO == PRO_BF16 || PRO == PRO_RMSNORM)
-        if (mode == M1_SWIGLU) return m1_pick_mode<F, PRO, M1_SWIGLU, 1>(ts, ntt, cpl, kc, senc, exact);
-    if (mode == M1_PLAIN) return m1_pick_mode<F, PRO, M1_PLAIN, 1>(ts, ntt, cpl, kc, senc, exact);
+        if (mode == M1_SWIGLU) return m1_pick_mode<F, PRO, M1_SWIGLU, 1>(ts, ntt, cpl, senc, exact);
+    if (mode == M1_PLAIN) return m1_pick_mode<F, PRO, M1_PLAIN, 1>(ts, ntt, cpl, senc, exact);
     return nullptr;
 }
 
 // Kernels of format F with the quantize / int8 prologues and with the folded
 // rmsnorm / swiglu prologues (each defined in its own translation unit).
 template <int F>
-m1_fn m1_pick_plain(int ts, int ntt, int cpl, int kc, int senc, int mode, bool exact, int pro, int mr);
+m1_fn m1_pick_plain(int ts, int ntt, int cpl, int senc, int mode, bool exact, int pro, int mr);
 template <int F>
-m1_fn m1_pick_folded(int ts, int ntt, int cpl, int kc, int senc, int mode, bool exact, int pro, int mr);
+m1_fn m1_pick_folded(int ts, int ntt, int cpl, int senc, int mode, bool exact, int pro, int mr);
 
 #define VQ_M1_PLAIN(F)                                                                                         \
     template <>                                                                                                \
-    m1_fn m1_pick_plain<F>(int ts, int ntt, int cpl, int kc, int senc, int mode, bool exact, int pro, int mr) { \
-        return pro == PRO_INT8 ? m1_pick_pro<F, PRO_INT8>(ts, ntt, cpl, kc, senc, mode, exact, mr)               \
-                               : m1_pick_pro<F, PRO_BF16>(ts, ntt, cpl, kc, senc, mode, exact, mr);              \
+    m1_fn m1_pick_plain<F>(int ts, int ntt, int cpl, int senc, int mode, bool exact, int pro, int mr) { \
+        return pro == PRO_INT8 ? m1_pick_pro<F, PRO_INT8>(ts, ntt, cpl, senc, mode, exact, mr)               \
+                               : m1_pick_pro<F, PRO_BF16>(ts, ntt, cpl, senc, mode, exact, mr);              \
     }
 #define VQ_M1_FOLDED(F)                                                                                         \
     template <>                                                                                                 \
-    m1_fn m1_pick_folded<F>(int ts, int ntt, int cpl, int kc, int senc, int mode, bool exact, int pro, int mr) { \
-        return pro == PRO_SWIGLU ? m1_pick_pro<F, PRO_SWIGLU>(ts, ntt, cpl, kc, senc, mode, exact, mr)             \
-                                 : m1_pick_pro<F, PRO_RMSNORM>(ts, ntt, cpl, kc, senc, mode, exact, mr);           \
+    m1_fn m1_pick_folded<F>(int ts, int ntt, int cpl, int senc, int mode, bool exact, int pro, int mr) { \
+        return pro == PRO_SWIGLU ? m1_pick_pro<F, PRO_SWIGLU>(ts, ntt, cpl, senc, mode, exact, mr)             \
+                                 : m1_pick_pro<F, PRO_RMSNORM>(ts, ntt, cpl, senc, mode, exact, mr);           \
     }
 
 }  // namespace vq

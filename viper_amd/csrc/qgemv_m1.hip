@@ -1,38 +1,34 @@
 // Host side of the M = 1 GEMV: launch shape and dispatch.
-#include "qgemv_m1.h"
+#include "qgemv_stream.h"
 
 namespace vq {
 
-// kc: chunks per row of a masked exact tiling (M1_MASKED), else 0.
 struct M1Shape {
     int ts, ntt, cpl;
-    int kc = 0;
 };
 
 static m1_fn m1_kernel(int qtype, const M1Shape& sh, int senc, int mode, bool exact, int pro, int mr = 1) {
     const bool folded = pro == PRO_RMSNORM || pro == PRO_SWIGLU;
-    const int ts = sh.ts, ntt = sh.ntt, cpl = sh.cpl, kc = sh.kc;
+    const int ts = sh.ts, ntt = sh.ntt, cpl = sh.cpl;
     switch (qtype) {
         case VIPER_QTYPE_Q4_G64:
-            return folded ? m1_pick_folded<4>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr)
-                          : m1_pick_plain<4>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr);
+            return folded ? m1_pick_folded<4>(ts, ntt, cpl, senc, mode, exact, pro, mr)
+                          : m1_pick_plain<4>(ts, ntt, cpl, senc, mode, exact, pro, mr);
         case VIPER_QTYPE_Q5_G64:
-            return folded ? m1_pick_folded<5>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr)
-                          : m1_pick_plain<5>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr);
+            return folded ? m1_pick_folded<5>(ts, ntt, cpl, senc, mode, exact, pro, mr)
+                          : m1_pick_plain<5>(ts, ntt, cpl, senc, mode, exact, pro, mr);
         case VIPER_QTYPE_Q6_G64:
-            return folded ? m1_pick_folded<6>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr)
-                          : m1_pick_plain<6>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr);
+            return folded ? m1_pick_folded<6>(ts, ntt, cpl, senc, mode, exact, pro, mr)
+                          : m1_pick_plain<6>(ts, ntt, cpl, senc, mode, exact, pro, mr);
         default:
-            return folded ? m1_pick_folded<8>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr)
-                          : m1_pick_plain<8>(ts, ntt, cpl, kc, senc, mode, exact, pro, mr);
+            return folded ? m1_pick_folded<8>(ts, ntt, cpl, senc, mode, exact, pro, mr)
+                          : m1_pick_plain<8>(ts, ntt, cpl, senc, mode, exact, pro, mr);
     }
 }
 
-// A launch shape takes the exact-tiling kernels: TS * CPL chunks per row, or
-// a masked tiling's chunks per row, and a row's scales in whole 16-byte words.
-static bool m1_exact(const M1Shape& sh, int cpr, int ngr) {
-    return (cpr == sh.ts * sh.cpl || (sh.kc != 0 && cpr == sh.kc)) && ngr % 8 == 0;
-}
+// A launch shape takes the exact-tiling kernels: TS * CPL chunks per row and
+// a row's scales in whole 16-byte words.
+static bool m1_exact(const M1Shape& sh, int cpr, int ngr) { return cpr == sh.ts * sh.cpl && ngr % 8 == 0; }
 
 // Per-CU row load of a shape: ceil(ceil(N / rows) / CUs) * rows (rows per
 // workgroup are halved for the swiglu pair, whose workgroups also read the
@@ -50,7 +46,8 @@ static long m1_load(const M1Shape& sh, int N, int cus, bool pair = false) {
 // pass), then fewer chunk slots per lane (more lanes per row, so each lane's
 // dot chain after the weights arrive is shorter), then the smaller workgroup
 // (two 320-thread workgroups per CU beat one of 640 on the north-star shape:
-// each quantizes and passes its barrier on its own).  With no exact tiling:
+// each quantizes and passes its barrier on its own).  One row of any other K
+// takes the streaming kernel (st_shape).  MR > 1 rows with no exact tiling:
 // the smallest team covering a row in 10 slots per lane (longer rows loop over
 // segments of 64 lanes), workgroup size by row load, ties to more rows per
 // workgroup (fewer redundant activation quantizations).
@@ -87,20 +84,13 @@ static M1Shape m1_shape(int cpr, int N, int cus, int min_ntt, int noct, bool pai
         consider(c);
     }
     if (best.ntt != 0) return best;
-    // masked exact tilings (one row: not the multi-row shapes), in the same order
-    for (const auto& s : M1_MASKED) {
-        const M1Shape c{s[0], s[1], s[2], s[3]};
-        if (mr > 1 || c.kc != cpr || c.ntt < min_ntt || (pair && !m1_pair_ok(c.ts, c.ntt))) continue;
-        consider(c);
-    }
-    if (best.ntt != 0) return best;
+    if (mr == 1) return best;
     int ts = 8;
     while (ts < 64 && ts * 10 < cpr) ts *= 2;
     for (const auto& s : M1_SHAPES) {
         const M1Shape c{s[0], s[1], s[2]};
-        if (c.ts != ts || c.cpl != 10 || c.ntt < min_ntt || (pair && !m1_pair_ok(c.ts, c.ntt))) continue;
-        if (mr > 1 && !m1_mr_shape_ok(c.ts, c.ntt, c.cpl)) continue;
-        const long load = m1_load(c, N, cus, pair);
+        if (c.ts != ts || c.cpl != 10 || c.ntt < min_ntt || !m1_mr_shape_ok(c.ts, c.ntt, c.cpl)) continue;
+        const long load = m1_load(c, N, cus);
         if (best_load < 0 || load < best_load || (load == best_load && c.ntt > best.ntt)) {
             best = c;
             best_load = load;
@@ -180,11 +170,85 @@ bool m1_rows_pair(int qtype, int K, int M) {
     return m1_pairs<4>(m1_exact(sh, K / 32, K / 64), sh.ntt, m1_mr(M), PRO_BF16);
 }
 
-bool m1_folded_ok(int qtype, int K, int N) {
-    const int ck = qtype == VIPER_QTYPE_W8_G32 ? 16 : 32;
-    const int noct = K / 8;
-    const M1Shape sh = m1_shape(K / ck, N, device_cus(), (noct + M1_XS - 1) / M1_XS, noct);
-    return sh.ntt != 0 && lds_m1(qtype, K) <= (size_t)LDS_MAX;
+// The folded prologues hold the whole row after one load round.
+bool m1_folded_ok(int qtype, int K) { return K <= 20480 && lds_m1(qtype, K) <= (size_t)LDS_MAX; }
+
+// ------------------------------------------------------- streaming launches
+
+// Launch shape of the streaming kernel: teams, slots and rows per unit, units
+// per workgroup, workgroups per XCD (0: dispatch order) and workgroups per
+// matrix.
+struct StShape {
+    int ts, cpl, r, upw, gx, grid, nb[3];
+};
+
+static StShape st_shape(int qtype, int K, const int* n, int nouts, int cus) {
+    const int cpr = K / (qtype == VIPER_QTYPE_W8_G32 ? 16 : 32);
+    StShape s{};
+    s.ts = cpr <= 16 ? 8 : cpr <= 32 ? 16 : cpr <= 64 ? 32 : 64;
+    const int slots = (cpr + s.ts - 1) / s.ts;
+    s.cpl = slots > 10 ? 10 : slots;  // (every slot but the last full, see the kernel)
+    s.r = 1;
+    auto units = [&](int rows) { const int ur = 64 / s.ts * s.r; return (rows + ur - 1) / ur; };
+    auto total = [&] {
+        long u = 0;
+        for (int i = 0; i < nouts; ++i) u += units(n[i]);
+        return u;
+    };
+    // Two rows per unit where a row fills two slots of 64 lanes (the
+    // activation is then read from LDS once for both) and every wave still
+    // has a unit (Q4, K = 3520, N = 4096 / 11008: 3.70 / 6.85 -> 3.42 / 5.52 us;
+    // N = 1024: 2.51 -> 2.65 us, so not there).
+    if (s.ts == 64 && s.cpl == 2 && total() >= 10L * cus) s.r = 2;
+    const long u = total();
+    // One workgroup per CU, or two where there are enough units for both and
+    // the kernel's registers let two sit on a CU (at most 128 per lane): small
+    // tiles from 10 units per CU on (Q4, K = 2048, N = 8192 / 20000: 3.72 / 6.5
+    // -> 3.49 / 5.55 us; N = 4096, 8 units: 2.88 -> 3.01 us), larger ones from
+    // 24 on (K = 7168, N = 8192 / 3000: 7.55 / 4.15 -> 7.22 / 4.61 us).
+    const int wide = qtype == VIPER_QTYPE_Q5_G64 || qtype == VIPER_QTYPE_Q6_G64;  // high-plane registers
+    const bool two = s.cpl <= 2 ? u >= 10L * cus : s.cpl <= (wide ? 4 : 5) && u >= 24L * cus;
+    const long wgs = (two ? 2L : 1L) * cus;
+    long upw = (u + wgs - 1) / wgs;
+    s.upw = (int)(upw < 1 ? 1 : upw > 1023 ? 1023 : upw);
+    long g = 0;
+    for (int i = 0; i < nouts; ++i) {
+        s.nb[i] = (units(n[i]) + s.upw - 1) / s.upw;
+        g += s.nb[i];
+    }
+    s.gx = (int)((g + 7) / 8);
+    s.grid = 8 * s.gx;
+    if (s.gx > 1023) {
+        s.gx = 0;
+        s.grid = (int)g;
+    }
+    return s;
+}
+
+static m1_fn st_kernel(int qtype, const StShape& s, int senc, int mode, int pro) {
+    switch (qtype) {
+        case VIPER_QTYPE_Q4_G64: return st_pick<4>(s.ts, s.cpl, s.r, senc, mode, pro);
+        case VIPER_QTYPE_Q5_G64: return st_pick<5>(s.ts, s.cpl, s.r, senc, mode, pro);
+        case VIPER_QTYPE_Q6_G64: return st_pick<6>(s.ts, s.cpl, s.r, senc, mode, pro);
+        default: return st_pick<8>(s.ts, s.cpl, s.r, senc, mode, pro);
+    }
+}
+
+static size_t st_lds(int qtype, int K, const StShape& s) {
+    switch (qtype) {
+        case VIPER_QTYPE_Q4_G64: return st_lds_bytes<4>(K, s.ts * s.cpl);
+        case VIPER_QTYPE_Q5_G64: return st_lds_bytes<5>(K, s.ts * s.cpl);
+        case VIPER_QTYPE_Q6_G64: return st_lds_bytes<6>(K, s.ts * s.cpl);
+        default: return st_lds_bytes<8>(K, s.ts * s.cpl);
+    }
+}
+
+static int st_kw(int K, const StShape& s) { return (int)((unsigned)(K / 32) | (unsigned)s.upw << 12 | (unsigned)s.gx << 22); }
+
+// One row of this K takes an exact tiling of qgemv_m1_kernel.
+static bool m1_tiled(int qtype, int K) {
+    const bool w8 = qtype == VIPER_QTYPE_W8_G32;
+    return m1_tiles(w8 ? 8 : 4, K / (w8 ? 16 : 32));
 }
 
 int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa, float eps, void* xout,
@@ -201,66 +265,100 @@ int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa
         if (outs[i].n >= M1_N_EXTRA || ntot > INT32_MAX - outs[i].n) return VIPER_INVALID_ARGUMENT;
         ntot += outs[i].n;
     }
-    // The folded prologues hold the whole row after one load round, and run
-    // fastest with one octet per thread (rmsnorm's row sum and swiglu's
-    // element work are then a single pass): take such a workgroup when an
-    // exact tiling allows it, even at a higher row load.
     const int noct = M * (K / 8);
     const int cus = device_cus();
-    M1Shape sh{0, 0, 0};
-    if (folded) sh = m1_shape(K / ck, ntot, cus, noct < 640 ? noct : 640, noct);
-    if (sh.ntt == 0) {
-        const int min_ntt = mr > 1 ? (noct + M1_XS_MR - 1) / M1_XS_MR : folded ? (noct + M1_XS - 1) / M1_XS : 0;
-        sh = m1_shape(K / ck, ntot, cus, min_ntt, noct, false, mr);
-    }
-    if (sh.ntt == 0) return VIPER_INVALID_ARGUMENT;
-    if (!folded && nouts == 1 && mr == 1) sh = m1_q5_bf16(qtype, pro, ntot, cus, m1_wide96(qtype, K / ck, ntot, cus, sh));
-    const int group = qtype == VIPER_QTYPE_W8_G32 ? 32 : 64;
-    const bool exact = m1_exact(sh, K / ck, K / group);
-    const m1_fn fn = m1_kernel(qtype, sh, senc, part != nullptr ? M1_PART : M1_PLAIN, exact, pro, mr);
-    if (fn == nullptr) return VIPER_INTERNAL;
-    const int rows = sh.ntt / sh.ts;
-    const size_t lds = lds_m1_launch(qtype, K, rows, exact, mr);
-    if (lds > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
+    m1_fn fn;
+    unsigned grid, threads;
+    size_t lds;
     int nb[3] = {0, 0, 0};
-    for (int i = 0; i < nouts; ++i) nb[i] = (outs[i].n + rows - 1) / rows;
+    int kg;  // the K slot: streaming launches pack more into it, exact tilings carry the grid size
+    if (mr == 1 && !m1_tiled(qtype, K)) {
+        const int n[3] = {outs[0].n, nouts > 1 ? outs[1].n : 0, nouts > 2 ? outs[2].n : 0};
+        const StShape ss = st_shape(qtype, K, n, nouts, cus);
+        fn = st_kernel(qtype, ss, senc, part != nullptr ? M1_PART : M1_PLAIN, pro);
+        for (int i = 0; i < nouts; ++i) nb[i] = ss.nb[i];
+        grid = (unsigned)ss.grid;
+        threads = ST_NTT;
+        lds = st_lds(qtype, K, ss);
+        kg = st_kw(K, ss);
+    } else {
+        // The folded prologues run fastest with one octet per thread (rmsnorm's
+        // row sum and swiglu's element work are then a single pass): take such
+        // a workgroup where a tiling allows it, even at a higher row load.
+        M1Shape sh{0, 0, 0};
+        if (folded) sh = m1_shape(K / ck, ntot, cus, noct < 640 ? noct : 640, noct);
+        if (sh.ntt == 0)
+            sh = m1_shape(K / ck, ntot, cus, mr > 1 ? (noct + M1_XS_MR - 1) / M1_XS_MR : 0, noct, false, mr);
+        if (sh.ntt == 0) return VIPER_INVALID_ARGUMENT;
+        if (!folded && nouts == 1 && mr == 1) sh = m1_q5_bf16(qtype, pro, ntot, cus, m1_wide96(qtype, K / ck, ntot, cus, sh));
+        const int group = qtype == VIPER_QTYPE_W8_G32 ? 32 : 64;
+        const bool exact = m1_exact(sh, K / ck, K / group);
+        fn = m1_kernel(qtype, sh, senc, part != nullptr ? M1_PART : M1_PLAIN, exact, pro, mr);
+        const int rows = sh.ntt / sh.ts;
+        lds = lds_m1_launch(qtype, K, rows, exact, mr);
+        if (lds > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
+        for (int i = 0; i < nouts; ++i) nb[i] = (outs[i].n + rows - 1) / rows;
+        grid = (unsigned)(nb[0] + nb[1] + nb[2]);
+        threads = (unsigned)sh.ntt;
+        kg = exact ? (int)grid : K;
+    }
+    if (fn == nullptr) return VIPER_INTERNAL;
     const M1Out o0 = outs[0], o1 = nouts > 1 ? outs[1] : outs[0], o2 = nouts > 2 ? outs[2] : outs[0];
     const uint8_t *w0 = (const uint8_t*)o0.w, *w1 = (const uint8_t*)o1.w, *w2 = (const uint8_t*)o2.w;
     const uint16_t *s0 = (const uint16_t*)o0.s, *s1 = (const uint16_t*)o1.s, *s2 = (const uint16_t*)o2.s;
     uint16_t *y0 = (uint16_t*)o0.y, *y1 = (uint16_t*)o1.y, *y2 = (uint16_t*)o2.y;
-    int n0 = o0.n | (pro == PRO_RMSNORM && xout != nullptr ? M1_N_EXTRA : 0), n1 = o1.n, n2 = o2.n;
+    int n0 = o0.n | (pro == PRO_RMSNORM && xout != nullptr ? M1_N_EXTRA : 0);
+    int n1 = nouts > 1 ? o1.n : 0, n2 = nouts > 2 ? o2.n : 0;
     int e0 = nb[0], e1 = nb[0] + nb[1];
     if (mr > 1) e1 = M;  // one matrix: e1 carries the activation rows
-    const unsigned grid = (unsigned)(nb[0] + nb[1] + nb[2]);
     const uint16_t* r = (const uint16_t*)res;
-    // an exact tiling's K is a kernel constant: the slot carries the grid size
-    int kg = exact ? (int)grid : K;
     void* args[] = {&x, &w0, &s0, &y0, &kg, &n0, &e0, &e1, &r, &xa, &eps, &xout, &part,
                     &w1, &s1, &y1, &n1, &w2, &s2, &y2, &n2};
-    launch((const void*)fn, grid, (unsigned)sh.ntt, lds, st, args);
+    launch((const void*)fn, grid, threads, lds, st, args);
     return status_of(hipGetLastError());
 }
 
 int launch_m1_timeline(int qtype, int senc, int K, const void* x, const void* w, const void* s, void* y, int N,
                        uint64_t* stamps, size_t stamp_bytes, int* workgroups, int* waves, hipStream_t st) {
+    // rows that TS x CPL lanes and slots tile (5, 6 or 10 slots, or 336 chunks)
+    // and whose scales fill whole 16-byte words
     const int ck = qtype == VIPER_QTYPE_W8_G32 ? 16 : 32, group = qtype == VIPER_QTYPE_W8_G32 ? 32 : 64;
-    const int noct = K / 8;
+    const int cpr = K / ck;
+    if ((cpr != 80 && cpr != 160 && cpr != 320 && cpr != 640 && cpr != 96 && cpr != 192 && cpr != 384 && cpr != 336) ||
+        (K / group) % 8 != 0)
+        return VIPER_INVALID_ARGUMENT;
     const int cus = device_cus();
-    const M1Shape sh = m1_q5_bf16(qtype, PRO_BF16, N, cus, m1_wide96(qtype, K / ck, N, cus, m1_shape(K / ck, N, cus, 0, noct)));  // as launch_m1
-    if (sh.ntt == 0 || !m1_exact(sh, K / ck, K / group)) return VIPER_INVALID_ARGUMENT;
-    const m1_fn fn = m1_kernel(qtype, sh, senc, M1_TL, true, PRO_BF16);
+    m1_fn fn;
+    int nwg, threads, kg;  // as launch_m1
+    unsigned grid;
+    size_t lds;
+    if (m1_tiled(qtype, K)) {
+        const M1Shape sh = m1_q5_bf16(qtype, PRO_BF16, N, cus, m1_wide96(qtype, cpr, N, cus, m1_shape(cpr, N, cus, 0, K / 8)));
+        fn = m1_kernel(qtype, sh, senc, M1_TL, true, PRO_BF16);
+        const int rows = sh.ntt / sh.ts;
+        nwg = (N + rows - 1) / rows;
+        grid = (unsigned)nwg;
+        threads = sh.ntt;
+        lds = lds_m1_launch(qtype, K, rows, true);
+        kg = nwg;
+    } else {
+        const StShape ss = st_shape(qtype, K, &N, 1, cus);
+        fn = st_kernel(qtype, ss, senc, M1_TL, PRO_BF16);
+        nwg = ss.nb[0];
+        grid = (unsigned)ss.grid;
+        threads = ST_NTT;
+        lds = st_lds(qtype, K, ss);
+        kg = st_kw(K, ss);
+    }
     if (fn == nullptr) return VIPER_INTERNAL;
-    const int rows = sh.ntt / sh.ts;
-    const int grid = (N + rows - 1) / rows;
-    const size_t need = (size_t)grid * (sh.ntt / 64) * M1_TL_STAMPS * sizeof(uint64_t);
+    const size_t need = (size_t)nwg * (threads / 64) * M1_TL_STAMPS * sizeof(uint64_t);
     if (stamps == nullptr || stamp_bytes < need) return VIPER_INVALID_ARGUMENT;
-    if (workgroups != nullptr) *workgroups = grid;
-    if (waves != nullptr) *waves = sh.ntt / 64;
-    const size_t lds = lds_m1_launch(qtype, K, rows, true);
+    if (workgroups != nullptr) *workgroups = nwg;
+    if (waves != nullptr) *waves = threads / 64;
     const uint8_t* w0 = (const uint8_t*)w;
     const uint16_t* s0 = (const uint16_t*)s;
     uint16_t* y0 = (uint16_t*)y;
-    int kg = grid, n0 = N, e0 = grid, e1 = grid, nz = 0;
+    int n0 = N, e0 = nwg, e1 = nwg, nz = 0;
     const uint16_t* r = nullptr;
     const void* xa = nullptr;
     float eps = 0.0f;
@@ -269,7 +367,7 @@ int launch_m1_timeline(int qtype, int senc, int K, const void* x, const void* w,
     const void* nul = nullptr;
     void* args[] = {&x, &w0, &s0, &y0, &kg, &n0, &e0, &e1, &r, &xa, &eps, &xout, &part,
                     &nul, &nul, &nul, &nz, &nul, &nul, &nul, &nz};
-    launch((const void*)fn, (unsigned)grid, (unsigned)sh.ntt, lds, st, args);
+    launch((const void*)fn, grid, (unsigned)threads, lds, st, args);
     return status_of(hipGetLastError());
 }
 
@@ -281,23 +379,35 @@ int launch_m1_swiglu(int qtype, int senc, int K, int pro, const void* x, const v
     const int ck = qtype == VIPER_QTYPE_W8_G32 ? 16 : 32;
     const int noct = K / 8;
     const int cus = device_cus();
-    M1Shape sh{0, 0, 0};
-    if (pro == PRO_RMSNORM) sh = m1_shape(K / ck, N, cus, noct < 640 ? noct : 640, noct, true);
-    if (sh.ntt == 0) sh = m1_shape(K / ck, N, cus, pro == PRO_RMSNORM ? (noct + M1_XS - 1) / M1_XS : 0, noct, true);
-    if (sh.ntt == 0) return VIPER_INVALID_ARGUMENT;
-    const int group = qtype == VIPER_QTYPE_W8_G32 ? 32 : 64;
-    const bool exact = m1_exact(sh, K / ck, K / group);
-    const m1_fn fn = m1_kernel(qtype, sh, senc, M1_SWIGLU, exact, pro);
+    m1_fn fn;
+    unsigned grid, threads;
+    size_t lds;
+    int kg;  // as in launch_m1
+    if (!m1_tiled(qtype, K)) {
+        const StShape ss = st_shape(qtype, K, &N, 1, cus);
+        fn = st_kernel(qtype, ss, senc, M1_SWIGLU, pro);
+        grid = (unsigned)ss.grid;
+        threads = ST_NTT;
+        lds = st_lds(qtype, K, ss);
+        kg = st_kw(K, ss);
+    } else {
+        M1Shape sh{0, 0, 0};
+        if (pro == PRO_RMSNORM) sh = m1_shape(K / ck, N, cus, noct < 640 ? noct : 640, noct, true);
+        if (sh.ntt == 0) sh = m1_shape(K / ck, N, cus, 0, noct, true);
+        if (sh.ntt == 0) return VIPER_INVALID_ARGUMENT;
+        fn = m1_kernel(qtype, sh, senc, M1_SWIGLU, true, pro);
+        const int rows = sh.ntt / sh.ts;
+        grid = (unsigned)((N + rows / 2 - 1) / (rows / 2));
+        threads = (unsigned)sh.ntt;
+        lds = lds_m1_launch(qtype, K, rows, true);
+        kg = (int)grid;
+    }
     if (fn == nullptr) return VIPER_INTERNAL;
-    const int rows = sh.ntt / sh.ts;
-    const size_t lds = lds_m1_launch(qtype, K, rows, exact);
-    if (lds > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
     // every workgroup is a pair of gate and up rows; the up matrix goes in the
     // residual's slot (weights) and e0 / e1 (scales), the product to y0, the
     // optional gate / up outputs to y1 / y2 (flagged in n0)
     const bool extra = g_out != nullptr || u_out != nullptr || (pro == PRO_RMSNORM && xout != nullptr);
     int n0 = N | (extra ? M1_N_EXTRA : 0), n1 = N, n2 = N;
-    const unsigned grid = (unsigned)((N + rows / 2 - 1) / (rows / 2));
     const uint64_t su_bits = (uint64_t)(uintptr_t)su;
     int e0 = (int)(uint32_t)su_bits, e1 = (int)(uint32_t)(su_bits >> 32);
     const uint8_t *w0 = (const uint8_t*)wg, *w1 = nullptr, *w2 = nullptr;
@@ -305,10 +415,9 @@ int launch_m1_swiglu(int qtype, int senc, int K, int pro, const void* x, const v
     uint16_t *y0 = (uint16_t*)h, *y1 = (uint16_t*)g_out, *y2 = (uint16_t*)u_out;
     const uint16_t* r = (const uint16_t*)wu;
     int32_t* part = nullptr;
-    int kg = exact ? (int)grid : K;  // as in launch_m1
     void* args[] = {&x, &w0, &s0, &y0, &kg, &n0, &e0, &e1, &r, &xa, &eps, &xout, &part,
                     &w1, &s1, &y1, &n1, &w2, &s2, &y2, &n2};
-    launch((const void*)fn, grid, (unsigned)sh.ntt, lds, st, args);
+    launch((const void*)fn, grid, threads, lds, st, args);
     return status_of(hipGetLastError());
 }
 

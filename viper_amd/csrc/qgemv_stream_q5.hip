@@ -1,0 +1,8 @@
+// Streaming M = 1 GEMV kernels of format 5 (the template is in qgemv_stream.h).
+#include "qgemv_stream.h"
+
+namespace vq {
+
+VQ_ST_PICK(5)
+
+}  // namespace vq

@@ -7,7 +7,8 @@
 // kernels/ops/dp4a_smem_kernel.cu:25-74 and linear_multim.cu:64-130, weight
 // layout as tools/convert/convert.cpp:91-127.  The design is gfx950's own.
 //
-// M = 1 (qgemv_m1_kernel in qgemv_m1.h, the decode GEMV): teams of 16-64
+// M = 1 (the decode GEMV; qgemv_m1_kernel in qgemv_m1.h where its tilings fit
+// the row exactly, else qgemv_stream_kernel in qgemv_stream.h): teams of 8-64
 // lanes stream output rows with 16-byte non-temporal loads; each workgroup
 // quantizes the bf16 activation into LDS while its weights are in flight,
 // the int32 group dots are exact (v_dot8 on split activation nibbles for Q4,
@@ -568,7 +569,7 @@ extern "C" int viper_hip_qlinear_m1(int qtype, int scale_enc, int group, int K, 
         return VIPER_INVALID_ARGUMENT;
     if (norm_out != nullptr && prologue != VIPER_PROLOGUE_RMSNORM) return VIPER_INVALID_ARGUMENT;
     if (vq::lds_m1(qtype, K) > (size_t)vq::LDS_MAX) return VIPER_INVALID_ARGUMENT;
-    if ((prologue == VIPER_PROLOGUE_RMSNORM || prologue == VIPER_PROLOGUE_SWIGLU) && !vq::m1_folded_ok(qtype, K, N[0]))
+    if ((prologue == VIPER_PROLOGUE_RMSNORM || prologue == VIPER_PROLOGUE_SWIGLU) && !vq::m1_folded_ok(qtype, K))
         return VIPER_INVALID_ARGUMENT;
     return vq::launch_m1(qtype, scale_enc, K, prologue, a, b, eps, norm_out, outs, n_out, residual_bf16, nullptr,
                          (hipStream_t)stream);
@@ -589,7 +590,7 @@ extern "C" int viper_hip_qlinear_m1_swiglu(int qtype, int scale_enc, int group, 
     if (vq::misaligned(a, 16) || vq::misaligned(b, 16) || vq::misaligned(norm_out, 16)) return VIPER_INVALID_ARGUMENT;
     if (norm_out != nullptr && prologue != VIPER_PROLOGUE_RMSNORM) return VIPER_INVALID_ARGUMENT;
     if (vq::lds_m1(qtype, K) > (size_t)vq::LDS_MAX) return VIPER_INVALID_ARGUMENT;
-    if (prologue == VIPER_PROLOGUE_RMSNORM && !vq::m1_folded_ok(qtype, K, N)) return VIPER_INVALID_ARGUMENT;
+    if (prologue == VIPER_PROLOGUE_RMSNORM && !vq::m1_folded_ok(qtype, K)) return VIPER_INVALID_ARGUMENT;
     return vq::launch_m1_swiglu(qtype, scale_enc, K, prologue, a, b, eps, norm_out, w_gate, s_gate, w_up, s_up, N,
                                 h_bf16, gate_bf16, up_bf16, (hipStream_t)stream);
 }

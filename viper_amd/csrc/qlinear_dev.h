@@ -89,6 +89,22 @@ __device__ __forceinline__ int group_sum(int v) {
     return v;
 }
 
+// The last steps of a team's sum: over the 16-lane rows of the wave, with
+// the lane-swap instructions (no LDS round trip, as a permute through it
+// would take).
+template <int TS>
+__device__ __forceinline__ float team_sum_rows(float v) {
+    if constexpr (TS >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    if constexpr (TS >= 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    return v;
+}
+
 // Sum over a team of TS consecutive lanes; every lane of the team gets it.
 template <int TS>
 __device__ __forceinline__ float team_sum(float v) {
@@ -96,9 +112,7 @@ __device__ __forceinline__ float team_sum(float v) {
     if constexpr (TS >= 4) v += dpp_f<DPP_SWAP2>(v);
     if constexpr (TS >= 8) v += dpp_f<DPP_HALF_MIRROR>(v);
     if constexpr (TS >= 16) v += dpp_f<DPP_MIRROR>(v);
-    if constexpr (TS >= 32) v += __shfl_xor(v, 16, 64);
-    if constexpr (TS >= 64) v += __shfl_xor(v, 32, 64);
-    return v;
+    return team_sum_rows<TS>(v);
 }
 
 // Logical block of workgroup b in a grid of g: the dispatcher deals

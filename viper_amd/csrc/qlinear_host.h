@@ -90,7 +90,7 @@ struct M1Out {
     int n;
 };
 size_t lds_m1(int qtype, int K);
-bool m1_folded_ok(int qtype, int K, int N);
+bool m1_folded_ok(int qtype, int K);
 // M (1..4) activation rows: M > 1 needs one matrix, PRO_BF16 or PRO_INT8 and
 // m1_rows_ok (x, y, res and part hold M rows).
 int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa, float eps, void* xout,
