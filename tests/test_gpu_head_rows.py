@@ -1,0 +1,45 @@
+"""GPU parity of the LM head's matrix-core kernel (several activation rows) at the edges of its tiles: rows of the last
+tile, one to many tiles per wave, row lengths around a 512-byte segment and a 16-byte chunk, every row count that picks
+it, non-finite weights and activations staying in their own row and column."""
+import numpy as np
+import pytest
+
+import oracle as O
+import viper_amd as va
+from test_gpu_lm_head import bf16, dev, host_u16, torch_dev  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def run(torch, w, x):
+    M, N = x.shape[0], w.shape[0]
+    y = torch.full((M, N), 7, dtype=torch.int16, device="cuda")
+    assert va.linear_bf16(dev(torch, w), dev(torch, x), y).ok()
+    torch.cuda.synchronize()
+    return host_u16(y)
+
+
+@pytest.mark.parametrize("M,N,K", [(5, 1, 8), (16, 15, 64), (7, 16, 248), (8, 17, 256), (6, 129, 264), (12, 1000, 2560),
+                                   (16, 4097, 2048), (3, 700, 4096), (4, 333, 2568), (2, 65, 16384), (9, 40000, 72),
+                                   (5, 12345, 512)])
+def test_head_rows(torch_dev, M, N, K):  # noqa: F811
+    rng = np.random.default_rng(7 * N + K + M)
+    w = bf16(0.05 * rng.standard_normal((N, K)))
+    x = O.gen_act(M, K, 0x4EAD + K)
+    y_ref, _, absterm = O.linear_bf16(w, x)
+    # fp32 sums in another order: 1e-5 of the sum of magnitudes covers K * 2^-24 for K up to 16384 (9.8e-4 * 1e-2)
+    O.assert_bf16_close(run(torch_dev, w, x), y_ref, absterm, rel=1e-5)
+
+
+def test_head_rows_nonfinite(torch_dev):  # noqa: F811
+    M, N, K = 8, 100, 1000
+    rng = np.random.default_rng(3)
+    w, x = bf16(0.05 * rng.standard_normal((N, K))), O.gen_act(M, K, 0x4EAE)
+    clean = run(torch_dev, w, x)
+    w[41, 999], x[3, 0] = 0x7F80, 0x7FC0  # +inf in one weight row, NaN in one activation row
+    y = O.bf16_to_f32(run(torch_dev, w, x))
+    assert np.isnan(y[3]).all()
+    assert not np.isfinite(y[:, 41]).any()
+    keep = np.ones((M, N), dtype=bool)
+    keep[3], keep[:, 41] = False, False
+    np.testing.assert_array_equal(y[keep], O.bf16_to_f32(clean)[keep])

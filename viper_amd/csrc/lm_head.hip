@@ -8,7 +8,8 @@
 // chunks of the row at once (non-temporal loads), after the activation loads
 // (loads retire in issue order, so x is staged into LDS while the weights
 // are in flight).  Each 16-byte chunk is 8 bf16 and costs 4 v_dot2_f32_bf16
-// per activation row; teams are reduced with DPP in a fixed order.
+// per activation row; teams are reduced with DPP in a fixed order.  More rows
+// take the matrix-core kernel below (head_mfma_kernel).
 //
 // Argmax: one workgroup per logits row; every lane requests all of its
 // 16-byte octets at once, keeps the first octet holding its largest value
@@ -106,6 +107,150 @@ gemv_bf16_kernel(const uint16_t* __restrict__ w, const uint16_t* x, uint16_t* __
         if (m < M) {
             const float v = team_sum<TS>(acc[m]);
             if (l == 0 && row_ok) y[(size_t)m * N + row] = f2bf(v);
+        }
+    }
+}
+
+// More rows on the matrix cores.  The dot kernel reads every activation row
+// from LDS for each weight chunk, so at 8 rows it is bound by LDS (166144 x
+// 2560: 117 us for 2 rows, 240 for 8, 455 for 12).  Here a weight tile of 16
+// rows is the A operand of v_mfma_f32_16x16x32_bf16 and the activation rows
+// the 16 columns of B, read once per tile.  A fragment load straight from
+// memory (16 rows x 64 bytes per instruction) streams at 4.9 TB/s, so each
+// wave loads 2 rows x 512 contiguous bytes per instruction and turns its 16
+// rows x 512 bytes through an LDS buffer of its own (row stride 528 bytes:
+// conflict-free 16-byte reads).  Persistent workgroups stage the activation
+// once; each wave keeps the next 8 KB segment (of the next tile, too) in
+// flight while it multiplies one.  Bound by the weight stream: 127 us for 2..6
+// rows, 129 for 8, 132 for 12 (850 MB, 6.5-6.7 TB/s; the dot kernel's one row
+// 117 us).  tpw tiles per workgroup: an odd number, about three workgroups per
+// CU (131072 x 4096: 157 us; 256 workgroups, whose first rows then lie 4 MB
+// apart and meet in the same memory channels, 178 us).
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int HM_NTT = 512;
+constexpr int HM_SC = 32;              // 16-byte chunks of a row per segment
+constexpr int HM_STR = HM_SC * 16 + 16;  // LDS row stride of the wave's buffer
+constexpr int HM_XS = LDS_MAX / 16 / HM_NTT;  // activation chunks per thread (at most 64 KiB of rows)
+
+__host__ __device__ constexpr size_t hm_lds_bytes(int M, int K) {
+    return (size_t)((K / 8 + HM_SC - 1) / HM_SC * HM_SC) * M * 16 + (size_t)(HM_NTT / 64) * 16 * HM_STR;
+}
+
+__global__ void __launch_bounds__(HM_NTT)
+head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N, int K, int tpw, int gx) {
+    constexpr int W = HM_NTT / 64, RI = 64 / HM_SC;
+    extern __shared__ __align__(16) u32x4 lx[];  // x as [chunk][M], zeros past the row; then the waves' buffers
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l16 = lane & 15, q = lane >> 4;
+    const int CPR = K / 8, NS = (CPR + HM_SC - 1) / HM_SC, KP = NS * HM_SC;
+    uint8_t* tb = (uint8_t*)(lx + (size_t)KP * M) + wave * (16 * HM_STR);
+    // workgroup blocks in XCD order; a grid rounded up to whole XCD turns
+    const int bid = ((int)blockIdx.x & 7) * gx + ((int)blockIdx.x >> 3);
+    const int tend = min((bid + 1) * tpw, (N + 15) / 16);
+    if (bid * tpw >= tend) return;
+    const int nx = M * CPR;
+    const auto xr = buf(x, (uint32_t)nx * 16);
+    u32x4 xv[HM_XS];
+#pragma unroll
+    for (int i = 0; i < HM_XS; ++i) xv[i] = bload16(xr, (tid + HM_NTT * i) * 16);
+    issue_fence();
+
+    struct Seg {
+        u32x4 v[16 / RI];
+    };
+    struct Cur {
+        int t, s;  // tile, segment of the row
+    };
+    const uint32_t rbytes = (uint32_t)K * 2;
+    auto advance = [&](Cur& c) {
+        if (++c.s == NS) {
+            c.s = 0;
+            c.t += W;
+        }
+    };
+    auto load = [&](Seg& S, const Cur& c) {
+        const int row0 = c.t * 16, n = min(16, N - row0);
+        const auto wr = buf(w + (size_t)row0 * K, (uint32_t)n * rbytes);
+        const int ch = c.s * HM_SC + lane % HM_SC;
+#pragma unroll
+        for (int i = 0; i < 16 / RI; ++i)
+            S.v[i] = bload16<AUX_NT>(wr, ch < CPR ? (i * RI + lane / HM_SC) * (int)rbytes + ch * 16 : OOB);
+    };
+    Cur lc{bid * tpw + wave, 0}, cc = lc;
+    Seg S0, S1;
+    if (lc.t < tend) load(S0, lc);
+    issue_fence();
+#pragma unroll
+    for (int i = 0; i < HM_XS; ++i) {
+        const int t = tid + HM_NTT * i;
+        if (t < nx) {
+            const int m = t / CPR, c = t - m * CPR;
+            lx[c * M + m] = xv[i];
+        }
+    }
+    for (int t = nx + tid; t < KP * M; t += HM_NTT) lx[t] = u32x4{0u, 0u, 0u, 0u};
+    lds_barrier();
+
+    const int mr = min(l16, M - 1);  // columns past M repeat the last row and are not stored
+    f32x4 a0 = {0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+    auto compute = [&](const Seg& S, const Cur& c) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < 16 / RI; ++i)
+            *(u32x4*)(tb + (i * RI + lane / HM_SC) * HM_STR + (lane % HM_SC) * 16) = S.v[i];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+        // k-slot q of each product: chunk q of its four (the same for both operands)
+#pragma unroll
+        for (int kb = 0; kb < HM_SC / 8; ++kb) {
+            const u32x4 w0 = *(const u32x4*)(tb + l16 * HM_STR + (kb * 8 + q) * 16);
+            const u32x4 w1 = *(const u32x4*)(tb + l16 * HM_STR + (kb * 8 + 4 + q) * 16);
+            const u32x4 x0 = lx[(c.s * HM_SC + kb * 8 + q) * M + mr], x1 = lx[(c.s * HM_SC + kb * 8 + 4 + q) * M + mr];
+            a0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w0), __builtin_bit_cast(bf16x8, x0),
+                                                         a0, 0, 0, 0);
+            a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w1), __builtin_bit_cast(bf16x8, x1),
+                                                         a1, 0, 0, 0);
+        }
+        if (c.s + 1 < NS) return;
+        // the lane holds rows 4q .. 4q + 3 of the tile for activation row l16
+        const int n0 = c.t * 16 + 4 * q;
+        const uint32_t p0 = f2bf2(a0[0] + a1[0], a0[1] + a1[1]), p1 = f2bf2(a0[2] + a1[2], a0[3] + a1[3]);
+        if (l16 < M) {
+            uint16_t* o = y + (size_t)l16 * N + n0;
+            if (n0 < N) o[0] = (uint16_t)p0;
+            if (n0 + 1 < N) o[1] = (uint16_t)(p0 >> 16);
+            if (n0 + 2 < N) o[2] = (uint16_t)p1;
+            if (n0 + 3 < N) o[3] = (uint16_t)(p1 >> 16);
+        }
+        a0 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        a1 = a0;
+    };
+    // (separate code for the last segment, so that no wait counts loads that
+    // may not have been issued)
+    if (cc.t < tend) {
+        for (;;) {
+            advance(lc);
+            if (lc.t >= tend) {
+                compute(S0, cc);
+                break;
+            }
+            load(S1, lc);
+            issue_fence();
+            compute(S0, cc);
+            advance(cc);
+            advance(lc);
+            if (lc.t >= tend) {
+                compute(S1, cc);
+                break;
+            }
+            load(S0, lc);
+            issue_fence();
+            compute(S1, cc);
+            advance(cc);
         }
     }
 }
@@ -292,8 +437,7 @@ template <int TS, bool EXACT>
 static lh_fn lh_pick_mt(int mt) {
     switch (mt) {
         case 1: return gemv_bf16_kernel<TS, 256, 1, EXACT>;
-        case 4: return gemv_bf16_kernel<TS, 256, 4, EXACT>;
-        default: return gemv_bf16_kernel<TS, 256, 16, EXACT>;
+        default: return gemv_bf16_kernel<TS, 256, 4, EXACT>;
     }
 }
 template <int TS>
@@ -311,11 +455,26 @@ extern "C" int viper_hip_linear_bf16(const void* w_bf16, const void* x_bf16, voi
         return VIPER_INVALID_ARGUMENT;
     const size_t lds = (size_t)M * K * 2;
     if (lds > (size_t)vq::LDS_MAX || (size_t)K * 2 * 256 > (size_t)INT32_MAX) return VIPER_INVALID_ARGUMENT;
+    // The dot kernel for one row and for the few whose LDS reads hide behind
+    // the weights (M x K up to 4 x 2560: 121 us against 127 on the matrix
+    // cores; 3 rows of 4096: 163 against 157; 5 rows of 1024: 43.7 against 40.2).
+    if (M > 4 || (M > 1 && M * K > 10240)) {
+        const int tiles = (N + 15) / 16, waves = vq::HM_NTT / 64;
+        int tpw = (tiles + 3 * vq::device_cus() - 1) / (3 * vq::device_cus());
+        if (tpw < waves) tpw = waves;  // a tile for every wave
+        tpw |= 1;
+        const int blocks = (tiles + tpw - 1) / tpw;
+        int gx = (blocks + 7) / 8;
+        void* args[] = {&w_bf16, &x_bf16, &y_bf16, &M, &N, &K, &tpw, &gx};
+        (void)hipLaunchKernel((const void*)vq::head_mfma_kernel, dim3((unsigned)(8 * gx)), dim3(vq::HM_NTT), args,
+                              vq::hm_lds_bytes(M, K), (hipStream_t)stream);
+        return vq::status_of(hipGetLastError());
+    }
     const int cpr = K / 8;
     int ts = 8;
     while (ts < 64 && ts * vq::LH_CPL < cpr) ts *= 2;
     const bool exact = cpr == ts * vq::LH_CPL;
-    const int mt = M == 1 ? 1 : M <= 4 ? 4 : 16;
+    const int mt = M == 1 ? 1 : 4;
     vq::lh_fn fn;
     switch (ts) {
         case 8: fn = vq::lh_pick<8>(mt, exact); break;

@@ -186,8 +186,9 @@ static StShape st_shape(int qtype, int K, const int* n, int nouts, int cus) {
     const int cpr = K / (qtype == VIPER_QTYPE_W8_G32 ? 16 : 32);
     StShape s{};
     s.ts = cpr <= 16 ? 8 : cpr <= 32 ? 16 : cpr <= 64 ? 32 : 64;
-    const int slots = (cpr + s.ts - 1) / s.ts;
-    s.cpl = slots > 10 ? 10 : slots;  // (every slot but the last full, see the kernel)
+    const bool wide = qtype == VIPER_QTYPE_Q5_G64 || qtype == VIPER_QTYPE_Q6_G64;  // high-plane registers
+    const int slots = (cpr + s.ts - 1) / s.ts, most = wide ? ST_MAX<5> : ST_MAX<4>;
+    s.cpl = slots > most ? most : slots;  // (every slot but the last full, see the kernel)
     s.r = 1;
     auto units = [&](int rows) { const int ur = 64 / s.ts * s.r; return (rows + ur - 1) / ur; };
     auto total = [&] {
@@ -206,7 +207,6 @@ static StShape st_shape(int qtype, int K, const int* n, int nouts, int cus) {
     // tiles from 10 units per CU on (Q4, K = 2048, N = 8192 / 20000: 3.72 / 6.5
     // -> 3.49 / 5.55 us; N = 4096, 8 units: 2.88 -> 3.01 us), larger ones from
     // 24 on (K = 7168, N = 8192 / 3000: 7.55 / 4.15 -> 7.22 / 4.61 us).
-    const int wide = qtype == VIPER_QTYPE_Q5_G64 || qtype == VIPER_QTYPE_Q6_G64;  // high-plane registers
     const bool two = s.cpl <= 2 ? u >= 10L * cus : s.cpl <= (wide ? 4 : 5) && u >= 24L * cus;
     const long wgs = (two ? 2L : 1L) * cus;
     long upw = (u + wgs - 1) / wgs;

@@ -18,7 +18,7 @@ namespace vq {
 // a second unit's loads in flight while it sums one; loads past its last unit
 // are not issued (an out-of-range load still takes the address unit's 16
 // clocks: issued anyway, they cost 0.5 us of a short launch).
-// K of more than TS * CPL chunks (shapes of 10 slots) is read in segments.
+// K of more than TS * CPL chunks (shapes of ST_MAX slots) is read in segments.
 //
 // What bounds it: the weight stream, once a launch is long (Q4, K = 11008,
 // N = 28672, 168 MB: 27.4-28.3 us, 6.0 TB/s); short ones the dispatch, the
@@ -40,6 +40,9 @@ constexpr int ST_NTT = 512;  // threads per workgroup
 // Weight-issue delay, s_sleep units, as in qgemv_m1_kernel (0 and 2 equal; 6
 // 0.05-0.1 us slower: only one unit per wave goes out ahead of the quantize).
 constexpr int ST_DELAY = 2;
+// Most chunk slots per lane (two units of more of Q5 / Q6 pass 256 registers).
+template <int F>
+constexpr int ST_MAX = F == 5 || F == 6 ? 8 : 10;
 constexpr int ST_SCALE_LDS = 1024;  // wave-private scale block: 64 lanes x 16 bytes
 
 template <int F>
@@ -66,11 +69,11 @@ struct StTile {
 };
 
 // Activation octets per thread loaded ahead of the weights: the whole row of a
-// single-segment shape; rows of several segments (shapes of 10 slots) up to
-// K = 20480, the longest the folded prologues take.
+// single-segment shape; rows of several segments (shapes of ST_MAX slots) up
+// to K = 20480, the longest the folded prologues take.
 template <int F>
 __host__ __device__ constexpr int st_rounds(int ts, int cpl) {
-    return cpl == 10 ? 20480 / 8 / ST_NTT : (ts * cpl * Fmt<F>::CK / 8 + ST_NTT - 1) / ST_NTT;
+    return cpl == ST_MAX<F> ? 20480 / 8 / ST_NTT : (ts * cpl * Fmt<F>::CK / 8 + ST_NTT - 1) / ST_NTT;
 }
 
 // kw: K / 32 in bits 0..11, units per workgroup in bits 12..21, workgroups
@@ -96,8 +99,8 @@ qgemv_stream_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16
     constexpr int UR = 64 / TS * R, W = NTT / 64, SEGW = TS * CPL;
     // slots that lie inside the row on every lane: all but the last one, as the
     // team has no more lanes than st_shape's rule needs (none certain in the
-    // last segment of a longer row, shapes of 10 slots)
-    constexpr int FULL = CPL == 10 ? 0 : CPL - 1;
+    // last segment of a longer row, shapes of ST_MAX slots)
+    constexpr int FULL = CPL == ST_MAX<F> ? 0 : CPL - 1;
     constexpr int HB = FT::HIW * 4;
     constexpr int OPC = FT::CK / 8, OPG = FT::G / 8;
     const int K = (kw & 0xfff) * 32, upw = (kw >> 12) & 0x3ff, gx = (int)((unsigned)kw >> 22);
@@ -412,7 +415,8 @@ qgemv_stream_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16
 template <int F, int SENC, int MODE, int PRO>
 m1_fn st_kernel_v(int ts, int cpl, int r) {
 #define VQ_ST(TS_, CPL_, R_) \
-    if (ts == TS_ && cpl == CPL_ && r == R_) return qgemv_stream_kernel<F, TS_, CPL_, R_, SENC, MODE, PRO>;
+    if constexpr (CPL_ <= ST_MAX<F>)  \
+        if (ts == TS_ && cpl == CPL_ && r == R_) return qgemv_stream_kernel<F, TS_, CPL_, R_, SENC, MODE, PRO>;
     VQ_ST(8, 1, 1) VQ_ST(8, 2, 1) VQ_ST(16, 2, 1) VQ_ST(32, 2, 1) VQ_ST(64, 2, 1) VQ_ST(64, 2, 2) VQ_ST(64, 3, 1) VQ_ST(64, 4, 1)
     VQ_ST(64, 5, 1) VQ_ST(64, 6, 1) VQ_ST(64, 7, 1) VQ_ST(64, 8, 1) VQ_ST(64, 9, 1) VQ_ST(64, 10, 1)
 #undef VQ_ST

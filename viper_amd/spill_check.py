@@ -5,9 +5,7 @@ Compiles each translation unit for gfx950 with the compiler's resource-usage rem
 kernel whose scratch size is not zero.  A kernel that spills its registers to scratch pays a memory
 round trip per spilled value; the multi-row int8 GEMV once did so at every row load and ran 2.4x
 slower.  Exits 1 if a kernel outside the known set below uses scratch:
-  - qgemv_m1_kernel in its partials mode (MODE 1, the test entry viper_hip_qlinear_partials);
-  - qgemv_m1_kernel for Q6 on 640 threads without an exact tiling (8-24 bytes: every LDS operand of a
-    segment is read before the first dot, 2-6 registers past the 168-VGPR limit of 640 threads).
+  - qgemv_m1_kernel in its partials mode (MODE 1, the test entry viper_hip_qlinear_partials).
 Usage: spill_check.py HIPCC FLAGS... -- SOURCES...
 """
 import re
@@ -40,13 +38,9 @@ def demangle(names):
 
 
 def known(pretty):
-    # qgemv_m1_kernel<F, TS, NTT, CPL, SENC, MODE, EXACT, PRO, MR, DELAY, KC>
-    m = re.search(r"qgemv_m1_kernel<(\d+), (\d+), (\d+), (\d+), (\d+), (\d+), (true|false), (\d+), (\d+), (\d+), (\d+)>",
-                  pretty)
-    if not m:
-        return False
-    f, ntt, mode, exact = int(m.group(1)), int(m.group(3)), int(m.group(6)), m.group(7) == "true"
-    return mode == 1 or (f == 6 and ntt == 640 and not exact)
+    # qgemv_m1_kernel<F, TS, NTT, CPL, SENC, MODE, ...>
+    m = re.search(r"qgemv_m1_kernel<(\d+), (\d+), (\d+), (\d+), (\d+), (\d+),", pretty)
+    return m is not None and int(m.group(6)) == 1
 
 
 def main():
