@@ -104,6 +104,11 @@ static bool rc_split_shape(int qtype, int rows, int K, int cus, RcShape& s) {
     return fn != nullptr && rc_regs(fn) <= RC_SPLIT_MAX_REGS;
 }
 
+bool rc_split_capped(int qtype, int N, int K) {
+    const int sk = rc_split_parts(K / group_of(qtype) / 4);
+    return (long)sk * N > 16L * 6 * device_cus();
+}
+
 int rc_split_blocks(int qtype, int N, int K) {
     const int G = group_of(qtype);
     if (G == 0 || K % (4 * G) != 0 || K >= (1 << 27)) return 0;
@@ -137,6 +142,12 @@ static size_t rc_launch_lds(int qtype, const RcShape& sh, int K, int am) {
 static RcShape rc_launch_shape(int qtype, int rows_total, int K) {
     const int F = qtype == VIPER_QTYPE_W8_G32 ? 8 : qtype;
     return rc_shape(F, rows_total, K / group_of(qtype) / 4, device_cus());
+}
+
+bool rc_capped(int qtype, long rows_total, int K) {
+    const RcShape sh = rc_launch_shape(qtype, (int)(rows_total < 1 << 28 ? rows_total : 1 << 28), K);
+    const bool bounded = !sh.one || sh.qw > 1;  // fewer than 48 rows a workgroup
+    return bounded && rows_total > 8L * sh.rb * device_cus();
 }
 
 // RC_BF16: every row's octets in RC_XR rounds of the workgroup, and the

@@ -1,0 +1,93 @@
+// Host side of the streaming skinny GEMM (qgemm_stream.h): launch shape, and
+// the choice between it and the row-contiguous kernel (qgemm_rc.h).
+#include "qgemm_stream.h"
+
+namespace vq {
+
+// Groups per wave and phase, phases, and rows per workgroup: one workgroup per
+// CU, every CU the same rows (both matrices of a pair together), at most 1024
+// a workgroup so that the phases' row sums (64 bytes a row) fit LDS.
+struct SgLaunch {
+    int np, pg, rpw;
+    sg_fn fn;
+    size_t lds;
+};
+constexpr int SG_RPW_MAX = 1024;
+
+static long sg_rows(int N, bool pair) { return pair ? 2L * N : N; }
+
+static bool sg_launch(int qtype, long rows_total, int K, int M, int am, bool part, int senc, SgLaunch& l) {
+    const int F = qtype == VIPER_QTYPE_W8_G32 ? 8 : qtype, G = group_of(qtype), NG = K / G;
+    const int most = SG_W * 2 * sg_ni_max(F, am, part);
+    const long rpw = (rows_total + device_cus() - 1) / device_cus();
+    l.np = (NG + most - 1) / most;
+    l.pg = (NG + l.np - 1) / l.np;
+    l.rpw = (int)(rpw < SG_RPW_MAX ? rpw : SG_RPW_MAX);
+    const int gw = (l.pg + SG_W - 1) / SG_W;
+    const bool pack = M <= 8;
+    switch (qtype) {
+        case VIPER_QTYPE_Q4_G64: l.fn = sg_pick_q4(gw, am, pack, part, senc, &l.lds); break;
+        case VIPER_QTYPE_Q5_G64: l.fn = sg_pick_q5(gw, am, pack, part, senc, &l.lds); break;
+        case VIPER_QTYPE_Q6_G64: l.fn = sg_pick_q6(gw, am, pack, part, senc, &l.lds); break;
+        default: l.fn = sg_pick_w8(gw, am, pack, part, senc, &l.lds); break;
+    }
+    if (l.fn == nullptr) return false;
+    if (am == RC_BF16) l.lds += sg_act_lds(G, 8, NG);
+    else if (l.np > 1) l.lds += (size_t)l.rpw * 64;
+    return l.lds <= (size_t)device_lds_max();
+}
+
+// K fits the registers of one workgroup's waves.
+bool sg_one_phase(int qtype, int K, int am) {
+    const int F = qtype == VIPER_QTYPE_W8_G32 ? 8 : qtype;
+    return K / group_of(qtype) <= SG_W * 2 * sg_ni_max(F, am, false);
+}
+
+// RC_BF16: at most 8 rows (a workgroup's quantize of more costs more than the
+// quantize launch: K = 3520, N = 2560, Q4, M = 16: 8.3 us against 4.9 + 2.1),
+// one phase, every row's octet pairs in SG_XR rounds.
+bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair) {
+    if (M > 8 || (long)M * K > (long)SG_XR * 64 * SG_W * 16) return false;
+    SgLaunch l;
+    return sg_launch(qtype, sg_rows(N, pair), K, M, RC_BF16, false, 0, l) && l.np == 1;
+}
+
+// Which calls the streaming kernel takes: K that the row-contiguous kernel
+// cannot (not a multiple of four groups), and K whose row-contiguous kernel
+// holds fewer rows per CU than the call has (its two-quad and segment-loop
+// kernels, see rc_capped), where it ran the chip in several rounds of
+// workgroups (fragments, M = 16, us, row-contiguous / streaming: Q4 N = 10240
+// K = 4096 12.2 / 9.0, K = 5120 13.7 / 10.9, K = 6144 19.3 / 11.7; Q5
+// N = 10240 K = 4096 13.7 / 10.3; Q6 13.2 / 11.4; W8 N = 10240 K = 3072 16.3 /
+// 11.0; and where it holds them: Q4 N = 5120 K = 4096 6.4 / 6.8, K = 5120
+// 7.0 / 8.3, N = 10240 K = 3072 6.4 / 7.7).
+bool sg_takes(int qtype, int N, int K, bool pair) { return !rc_ok(qtype, K) || rc_capped(qtype, sg_rows(N, pair), K); }
+
+int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
+              int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1, hipStream_t st) {
+    const bool pair = w1 != nullptr;
+    if (M < 1 || M > 16 || (part != nullptr && am != RC_FRAG)) return VIPER_INTERNAL;
+    if (am == RC_BF16 && !sg_bf16_ok(qtype, N, K, M, pair)) return VIPER_INTERNAL;
+    // (the limit of the row-contiguous kernel's argument word, for every K of whole group pairs)
+    if (M >= 2 && (K / group_of(qtype)) % 2 == 0 && N >= (1 << 27)) return VIPER_INVALID_ARGUMENT;
+    SgLaunch l;
+    if (!sg_launch(qtype, sg_rows(N, pair), K, M, am, part != nullptr, senc, l)) return VIPER_INTERNAL;
+    const unsigned nb = ((unsigned)N + (unsigned)l.rpw - 1) / (unsigned)l.rpw * (pair ? 2u : 1u), gx = (nb + 7) / 8;
+    if (gx >= 1u << 20) return VIPER_INVALID_ARGUMENT;
+    const int8_t* a0 = (const int8_t*)xq;
+    const float* a1 = (const float*)xs;
+    const uint8_t* a2 = (const uint8_t*)w;
+    const uint16_t* a3 = (const uint16_t*)s;
+    uint16_t* a4 = (uint16_t*)y;
+    const uint16_t* a5 = (const uint16_t*)res;
+    const uint8_t* b0 = (const uint8_t*)w1;
+    const uint16_t* b1 = (const uint16_t*)s1;
+    uint16_t* b2 = (uint16_t*)y1;
+    unsigned kk = (unsigned)(K / 32) | (unsigned)(l.pg - 1) << 20;
+    unsigned rg = (unsigned)l.rpw | gx << 12, ms = (unsigned)(M - 1) | (senc ? 16u : 0u);
+    void* args[] = {&a0, &a1, &a2, &a3, &a4, &kk, &N, &rg, &ms, &a5, &part, &b0, &b1, &b2};
+    launch((const void*)l.fn, 8 * gx, 64 * SG_W, l.lds, st, args);
+    return status_of(hipGetLastError());
+}
+
+}  // namespace vq

@@ -1,0 +1,10 @@
+// Streaming skinny-GEMM kernels of format 4 (the template is in qgemm_stream.h).
+#include "qgemm_stream.h"
+
+namespace vq {
+
+sg_fn sg_pick_q4(int gw, int am, bool pack, bool part, int senc, size_t* lds) {
+    return sg_pick<4>(gw, am, pack, part, senc, lds);
+}
+
+}  // namespace vq

@@ -162,6 +162,11 @@ bool m1_rows_ok(int qtype, int K, int M) {
     return sh.ntt != 0 && lds_m1_launch(qtype, K, 0, false, m1_mr(M)) + kBlockMax <= (size_t)LDS_MAX;
 }
 
+bool m1_rows_exact(int qtype, int K, int M) {
+    const bool w8 = qtype == VIPER_QTYPE_W8_G32;
+    return m1_rows_ok(qtype, K, M) && m1_tiles(w8 ? 8 : 4, K / (w8 ? 16 : 32));
+}
+
 bool m1_rows_pair(int qtype, int K, int M) {
     // the multi-row shape stages its rows two octets per thread (m1_pairs)
     if (qtype != VIPER_QTYPE_Q4_G64 || !m1_rows_ok(qtype, K, M)) return false;

@@ -15,10 +15,10 @@
 // v_dot4 on offset codes for Q5/Q6/W8) and the fp32 combine is reduced with
 // DPP in a fixed order (deterministic).
 //
-// M = 2..16 (qgemm_rc.h, qgemm_mfma.hip, qgemm_pre.hip): activations are
-// quantized once into a caller workspace (quantize_frag64_kernel in the
-// matrix-core fragment order, else quantize_act_kernel) or supplied by the
-// caller, and every weight byte is read once for all M rows.
+// M = 2..16 (qgemm_rc.h, qgemm_stream.h): few rows are quantized by every
+// workgroup, more are quantized once into a caller workspace in the
+// matrix-core fragment order or supplied by the caller, and every weight byte
+// is read once for all M rows.
 //
 // The activation quantizer never divides per element: with s the group scale
 // (an IEEE divide amax/127, once per group) and r = rcp(s) (the hardware
@@ -269,6 +269,27 @@ static int validate_second(const Second& b, int qtype, int senc, int group, int 
     return validate_weights(qtype, b.w, b.s, senc, group, N, K, M);
 }
 
+// Two to four rows of one matrix: on the M = 1 kernel's dot path, or on the
+// matrix cores?  The dot path's exact tilings (K = 2560: 2 rows 3.6 us against
+// 4.2 at N = 2560), and K beyond one phase of the streaming kernel, where its
+// serial phases or a second launch cost more (one: K has one phase; Q4, 2
+// rows, N = 2560, dot / matrix cores: K = 9600 8.9 / 11.7; K = 6144 7.3 / 5.0,
+// K = 4096 6.9 / 4.1, K = 1984 5.5 / 4.0, K = 512 4.3 / 2.7; 4 rows K = 4096,
+// N = 10240 11.2 / 9.0).  Two rows of the formats that decode cheapest stay on
+// the dots also where short rows are many (K = 2048, N = 20480: Q4 8.4 / 9.7,
+// W8 12.9 / 13.4; N = 8192 5.6 / 4.3, 6.8 / 6.7; K = 3520, where 40 rows per CU are
+// two and a half tiles, N = 10240: Q4 8.2 / 8.7) and where W8's kernel has its
+// most registers and one tile a workgroup (K = 3520, N = 2560 6.3 / 6.5;
+// N = 6144 11.0 / 9.7).
+static bool dot_rows(int qtype, int N, int K, int M, bool one) {
+    if (!m1_rows_ok(qtype, K, M)) return false;
+    if (m1_rows_exact(qtype, K, M) || !one) return true;
+    const bool w8 = qtype == VIPER_QTYPE_W8_G32;
+    const long per_cu = (N + (long)device_cus() - 1) / device_cus();
+    if (M > 2 || !(w8 || qtype == VIPER_QTYPE_Q4_G64)) return false;
+    return (per_cu > 32 && (K <= 2048 || (per_cu <= 48 && !rc_ok(qtype, K)))) || (w8 && K > 96 * 32 && !rc_ok(qtype, K) && per_cu <= 16);
+}
+
 static int qlinear_common(int qtype, const void* w, const void* s, int senc, int group, int N,
                           int K, const void* x, int M, void* y, const void* res, void* wsp,
                           size_t wsp_bytes, int32_t* part, void* stream, Second b = Second()) {
@@ -293,8 +314,10 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     // (north-star shape: M = 5 6.63 us, 8 7.49 us against 8.21 / 8.25 us for
     // the next-best path; at M >= 10 the rows' quantize in every workgroup
     // costs more than the quantize launch).
-    const bool mf = mfma_ok(qtype, K, M, s) && (b.w == nullptr || mfma_ok(qtype, K, M, b.s));
-    if (b.w == nullptr && M == 2 && m1_rows_ok(qtype, K, M)) {
+    const bool rc_k = M >= 2 && rc_ok(qtype, K);
+    const bool one = sg_bf16_ok(qtype, N, K, M, b.w != nullptr);
+    const bool dot = b.w == nullptr && dot_rows(qtype, N, K, M, one);
+    if (M == 2 && dot) {
         const M1Out outs[1] = {{w, s, y, N}};
         return launch_m1(qtype, senc, K, PRO_BF16, x, nullptr, 0.0f, nullptr, outs, 1, res, part, st, M);
     }
@@ -303,7 +326,11 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     // workgroup quantizing the bf16 rows of its own part of K, in one launch,
     // measured slower at every row count: down shape 3 / 8 / 16 rows 10.4 /
     // 12.6 / 15.9 us against 8.4 / 9.4 / 9.8 us.)
-    const bool split_ok = mf && b.w == nullptr && rc_split_blocks(qtype, N, K) > 0;
+    const bool split_ok = rc_k && b.w == nullptr && rc_split_blocks(qtype, N, K) > 0 && !rc_split_capped(qtype, N, K) && !one;
+    // K or rows beyond the row-contiguous kernel: the streaming one, which also
+    // quantizes up to 8 rows itself (Q4, M = 8, us, one launch / two: K = 3520,
+    // N = 2560 6.1 / 7.0, N = 10240 9.8 / 10.6; K = 4096, N = 10240 9.9 / 10.6).
+    const bool sg = !split_ok && sg_takes(qtype, N, K, b.w != nullptr);
     // Q5/Q6/W8 (K = 2560, N = 10240, 5% outlier channels): 3 or 4 rows of one
     // matrix run faster on the multi-row dot kernel below (Q5 4 rows 7.86
     // against 8.10 us; W8 3 / 4 rows 7.47 / 7.77 against 8.9 / 9.17 us); 5-8
@@ -311,8 +338,7 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     // (Q4 rows staged two octets per thread also past that size: down shape
     // K = 10240, 4 rows 8.4 us against 9.0-9.1 us for two launches with the K
     // split)
-    const bool rows_ok = b.w == nullptr && m1_rows_ok(qtype, K, M) &&
-                         ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M));
+    const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M));
     // With the rows staged two octets per thread (64-groups), the one-launch
     // path also wins for Q4 at 3-4 rows (5.45 / 5.74 against 5.6 / 5.9 us on the
     // dot kernel) and 9-10 rows (6.76 / 7.00 against 7.27 us in two launches;
@@ -321,7 +347,7 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     // rows on the dot kernel and 5-8 here.
     const bool q4 = qtype == VIPER_QTYPE_Q4_G64;
     const int bf_max = q4 && b.w == nullptr ? 10 : 8;
-    const bool bf_ok = mf && M >= 3 && M <= bf_max && !split_ok && rc_bf16_ok(qtype, N, K, M, b.w != nullptr);
+    const bool bf_ok = rc_k && !sg && M <= bf_max && !split_ok && rc_bf16_ok(qtype, N, K, M, b.w != nullptr);
     if (bf_ok && (M > 4 || !rows_ok || q4))
         return launch_rc(qtype, w, s, senc, N, K, x, nullptr, RC_BF16, M, y, res, part, b.w, b.s, b.y, st);
     // (3 or 4 rows here also where the LDS copy does not fit: while every
@@ -332,8 +358,10 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
         const M1Out outs[1] = {{w, s, y, N}};
         return launch_m1(qtype, senc, K, PRO_BF16, x, nullptr, 0.0f, nullptr, outs, 1, res, part, st, M);
     }
-    const bool staged = mf && mfma_staged(qtype, N, K);
-    if (!mf && lds_pre(qtype, M, K) > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
+    // one row or an odd number of groups: K has a limit
+    if ((M < 2 || (K / group_of(qtype)) % 2 != 0) && lds_pre(qtype, M, K) > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
+    if (sg && part == nullptr && one)
+        return launch_sg(qtype, w, s, senc, N, K, x, nullptr, RC_BF16, M, y, res, nullptr, b.w, b.s, b.y, st);
     const WsLayout lay = workspace_layout(qtype, N, K, M);
     if (split_ok && lay.blocks == 0) return VIPER_INTERNAL;
     uint8_t* xq = (uint8_t*)wsp + lay.xq;
@@ -343,15 +371,11 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     const bool split = split_ok;
     uint64_t* sp = split ? (uint64_t*)((uint8_t*)wsp + lay.sp) : nullptr;
     unsigned* sc = split ? (unsigned*)wsp : nullptr;
-    rc = launch_quantize(group, x, M, K, xq, xs, staged, st);
+    rc = launch_quantize(group, x, M, K, xq, xs, true, st);
     if (rc != VIPER_OK) return rc;
-    if (mf)
-        return launch_mfma(qtype, w, s, senc, N, K, xq, xs, !staged, M, y, res, part, b.w, b.s, b.y,
-                           st, sp, sc);
-    rc = launch_pre(qtype, w, s, senc, N, K, xq, xs, M, y, res, part, st);
-    if (rc == VIPER_OK && b.w != nullptr)
-        rc = launch_pre(qtype, b.w, b.s, senc, N, K, xq, xs, M, b.y, nullptr, nullptr, st);
-    return rc;
+    if (sg || !rc_k)
+        return launch_sg(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st);
+    return launch_rc(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st, sp, sc);
 }
 
 static int prequant_common(int qtype, const void* w, const void* s, int senc, int group, int N,
@@ -369,16 +393,17 @@ static int prequant_common(int qtype, const void* w, const void* s, int senc, in
         const M1Out outs[2] = {{w, s, y, N}, {b.w, b.s, b.y, N}};
         return launch_m1(qtype, senc, K, PRO_INT8, xq, xs, 0.0f, nullptr, outs, b.w ? 2 : 1, res, nullptr, st);
     }
-    if (b.w == nullptr && m1_rows_ok(qtype, K, M)) {
+    // (a K of whole group quads has no workgroup quantize here: on the matrix
+    // cores it is faster at many rows too, Q4 K = 2048, 2 rows, N = 10240 6.3 / 5.1)
+    if (b.w == nullptr && dot_rows(qtype, N, K, M, sg_one_phase(qtype, K, RC_NAT)) &&
+        (m1_rows_exact(qtype, K, M) || !sg_one_phase(qtype, K, RC_NAT) || !rc_ok(qtype, K))) {
         const M1Out outs[1] = {{w, s, y, N}};
         return launch_m1(qtype, senc, K, PRO_INT8, xq, xs, 0.0f, nullptr, outs, 1, res, nullptr, st, M);
     }
-    if (mfma_ok(qtype, K, M, s) && (b.w == nullptr || mfma_ok(qtype, K, M, b.s)))
-        return launch_mfma(qtype, w, s, senc, N, K, xq, xs, true, M, y, res, nullptr, b.w, b.s, b.y, st);
-    rc = launch_pre(qtype, w, s, senc, N, K, xq, xs, M, y, res, nullptr, st);
-    if (rc == VIPER_OK && b.w != nullptr)
-        rc = launch_pre(qtype, b.w, b.s, senc, N, K, xq, xs, M, b.y, nullptr, nullptr, st);
-    return rc;
+    if ((M < 2 || (K / group) % 2 != 0) && lds_pre(qtype, M, K) > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
+    if (M < 2 || sg_takes(qtype, N, K, b.w != nullptr))
+        return launch_sg(qtype, w, s, senc, N, K, xq, xs, RC_NAT, M, y, res, nullptr, b.w, b.s, b.y, st);
+    return launch_rc(qtype, w, s, senc, N, K, xq, xs, RC_NAT, M, y, res, nullptr, b.w, b.s, b.y, st);
 }
 
 // 2..16 int8 rows already in the matrix-core fragment order (a producer's
@@ -399,9 +424,11 @@ static int prequant_frag(int qtype, const void* w, const void* s, int senc, int 
     if (wsp != nullptr && misaligned(wsp, 16)) return VIPER_INVALID_ARGUMENT;
     const size_t need = b.w == nullptr ? frag_workspace_need(qtype, N, K, M) : 0;
     if (wsp != nullptr && need > 0 && wsp_bytes < need) return VIPER_INVALID_ARGUMENT;
-    const bool split = wsp != nullptr && need > 0;
+    const bool split = wsp != nullptr && need > 0 && !rc_split_capped(qtype, N, K);
     uint64_t* sp = split ? (uint64_t*)((uint8_t*)wsp + RC_CTL_BYTES) : nullptr;
     unsigned* sc = split ? (unsigned*)wsp : nullptr;
+    if (!split && sg_takes(qtype, N, K, b.w != nullptr))
+        return launch_sg(qtype, w, s, senc, N, K, xf, xsf, RC_FRAG, M, y, res, nullptr, b.w, b.s, b.y, (hipStream_t)stream);
     return launch_rc(qtype, w, s, senc, N, K, xf, xsf, RC_FRAG, M, y, res, nullptr, b.w, b.s, b.y,
                      (hipStream_t)stream, sp, sc);
 }

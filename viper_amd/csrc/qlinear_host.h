@@ -27,7 +27,8 @@ inline int group_of(int qtype) {
 
 inline size_t align16(size_t v) { return (v + 15) & ~(size_t)15; }
 
-// LDS of the prequantized kernel for M rows
+// Rows' quantized bytes, scales and chunk sums, for the limit on K of a call
+// whose K is an odd number of groups
 inline size_t lds_pre(int qtype, int M, int K) {
     const size_t G = (size_t)group_of(qtype);
     size_t b = (size_t)M * K + (size_t)M * (K / G) * 4;
@@ -96,6 +97,7 @@ bool m1_folded_ok(int qtype, int K);
 int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa, float eps, void* xout,
               const M1Out* outs, int nouts, const void* res, int32_t* part, hipStream_t st, int M = 1);
 bool m1_rows_ok(int qtype, int K, int M);
+bool m1_rows_exact(int qtype, int K, int M);
 // m1_rows_ok and the bf16 rows are staged two octets per thread (Q4, exact
 // tiling on 640 threads).
 bool m1_rows_pair(int qtype, int K, int M);
@@ -108,16 +110,6 @@ int launch_m1_timeline(int qtype, int senc, int K, const void* x, const void* w,
 int launch_m1_swiglu(int qtype, int senc, int K, int pro, const void* x, const void* xa, float eps, void* xout,
                      const void* wg, const void* sg, const void* wu, const void* su, int N, void* h, void* g_out,
                      void* u_out, hipStream_t st);
-
-// M <= 16 over prequantized activations, v_dot4 (qgemm_pre.hip).
-int launch_pre(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq,
-               const void* xs, int M, void* y, const void* res, int32_t* part, hipStream_t st);
-
-// M = 2..16 on the i8 matrix cores (qgemm_mfma.hip): needs K a multiple of
-// two groups and 4-byte aligned scales.  xnat: activations in the layout of
-// viper_hip_quantize_act, else in the fragment order quantize_act_kernel<G,
-// true> writes, which the shape must support (mfma_staged).
-bool mfma_ok(int qtype, int K, int M, const void* s);
 
 // M = 2..16, K a multiple of 4 groups (qgemm_rc.hip): row-contiguous weight
 // loads moved into the matrix-core layout through LDS.  am (RC_FRAG, RC_NAT,
@@ -158,12 +150,21 @@ int rc_split_blocks(int qtype, int N, int K);
 int launch_rc(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs,
               int am, int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1,
               hipStream_t st, uint64_t* sp = nullptr, unsigned* sc = nullptr);
-bool mfma_staged(int qtype, int N, int K);
+// The call's rows (both matrices of a pair) exceed what one workgroup per CU of
+// its row-contiguous kernel holds.
+bool rc_capped(int qtype, long rows_total, int K);
+// A split launch's (row, part) pairs exceed two workgroups of 48 rows per CU.
+bool rc_split_capped(int qtype, int N, int K);
 int launch_rc_timeline(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq,
                        const void* xs, int M, void* y, uint64_t* stamps, size_t stamp_bytes, int* workgroups,
                        int* waves, unsigned* sc, hipStream_t st);
-int launch_mfma(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq,
-                const void* xs, bool xnat, int M, void* y, const void* res, int32_t* part,
-                const void* w1, const void* s1, void* y1, hipStream_t st, uint64_t* sp = nullptr, unsigned* sc = nullptr);
+
+// M = 1..16, any K (qgemm_stream.hip): persistent workgroups, the activation
+// operands in registers.  am as for launch_rc; part only with RC_FRAG.
+bool sg_takes(int qtype, int N, int K, bool pair);
+bool sg_one_phase(int qtype, int K, int am);
+bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair);
+int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
+              int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1, hipStream_t st);
 
 }  // namespace vq
