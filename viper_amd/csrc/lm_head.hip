@@ -344,8 +344,8 @@ argmax_bf16_kernel(const uint16_t* logits, int32_t* __restrict__ out, int V) {
     }
 }
 
-// Split argmax: P workgroups per row, each over GR_OCT consecutive octets
-// (GR_NT threads, GR_OCT / GR_NT octets each, all requested at once), meet
+// Split argmax: P workgroups per row, each over GR_NT * PT consecutive octets
+// (GR_NT threads, PT octets each, all requested at once; greedy_octets), meet
 // through a 64-bit key per row in the caller's workspace:
 //   key = (order(value) << 32) | (0xFFFFFFFF - index),
 // where order maps floats to unsigned integers in the same order (+0 for
@@ -359,7 +359,6 @@ argmax_bf16_kernel(const uint16_t* logits, int32_t* __restrict__ out, int V) {
 // A workgroup with nothing above -inf offers (-inf, 0): a row with nothing
 // above -inf gives 0, as the single-workgroup kernel does.
 constexpr int GR_NT = 256;
-constexpr int GR_OCT = 512;  // octets (4096 logits, 8 KB) per workgroup
 
 __device__ __forceinline__ uint64_t greedy_key(float v, int i) {
     const uint32_t u = v == 0.0f ? 0u : __float_as_uint(v);
@@ -367,17 +366,18 @@ __device__ __forceinline__ uint64_t greedy_key(float v, int i) {
     return ((uint64_t)o << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)i);
 }
 
+template <int PT>
 __global__ void __launch_bounds__(GR_NT)
 argmax_split_kernel(const uint16_t* logits, int32_t* __restrict__ out, int V, int P, uint64_t* keys,
                     unsigned* cnt) {
     __shared__ float sv[GR_NT / 64];
     __shared__ int si[GR_NT / 64];
-    constexpr int PT = GR_OCT / GR_NT;
+    constexpr int OCT = GR_NT * PT;
     const int b = (int)blockIdx.x / P, p = (int)blockIdx.x % P;
     const int tid = (int)threadIdx.x;
     const int noct = V / 8;  // whole octets (the host takes this kernel for V % 8 == 0 only)
-    const int o0 = p * GR_OCT;
-    const int n = min(GR_OCT, noct - o0);
+    const int o0 = p * OCT;
+    const int n = min(OCT, noct - o0);
     const auto rr = buf(logits + (size_t)b * V + (size_t)o0 * 8, (uint32_t)n * 16);
     u32x4 q[PT];
 #pragma unroll
@@ -444,6 +444,18 @@ template <int TS>
 static lh_fn lh_pick(int mt, bool exact) {
     return exact ? lh_pick_mt<TS, true>(mt) : lh_pick_mt<TS, false>(mt);
 }
+
+// Octets per thread of the split argmax.  Every workgroup's two atomics go to
+// the one or two cache lines that hold all rows' keys and counters and are
+// performed one after another there, ~15 ns each: with two octets per thread
+// 166144 logits took 4.0 / 5.0 / 6.8 / 9.3 / 14.0 us for 1 / 2 / 4 / 8 / 16 rows,
+// with eight (a quarter of the workgroups) 4.1 / 4.1 / 4.5 / 5.0 / 6.0; 32000
+// logits 3.7 / 3.9 / 4.3 / 5.0 for 1 / 4 / 8 / 16 rows against 3.9 / 4.1 / 4.2 /
+// 4.2.  So eight from 49 workgroups of two octets on.  (512 threads of four or
+// eight octets 5.2 us for 8 rows, 1024 threads 5.8-6.3.)
+constexpr int GR_WGS = 48;
+static long greedy_wgs(int B, int V, int pt) { return (long)B * ((V / 8 + GR_NT * pt - 1) / (GR_NT * pt)); }
+static int greedy_octets(int B, int V) { return greedy_wgs(B, V, 2) > GR_WGS ? 8 : 2; }
 
 }  // namespace vq
 
@@ -517,13 +529,14 @@ extern "C" int viper_hip_sampling_greedy_split(const void* logits_bf16, int32_t*
     // rows that are not whole 16-byte octets take the one-workgroup kernel
     if (vq::misaligned(logits_bf16, 16) || V % 8 != 0)
         return viper_hip_sampling_greedy(logits_bf16, out_token, B, V, stream);
-    int P = (V / 8 + vq::GR_OCT - 1) / vq::GR_OCT;
-    if ((long)P * B > (long)INT32_MAX) return VIPER_INVALID_ARGUMENT;
+    if (vq::greedy_wgs(B, V, 2) > (long)INT32_MAX) return VIPER_INVALID_ARGUMENT;
+    const int pt = vq::greedy_octets(B, V);
+    int P = (int)vq::greedy_wgs(1, V, pt);
+    const void* fn = pt == 8 ? (const void*)vq::argmax_split_kernel<8> : (const void*)vq::argmax_split_kernel<2>;
     const uint16_t* a0 = (const uint16_t*)logits_bf16;
     uint64_t* keys = (uint64_t*)workspace;
     unsigned* cnt = (unsigned*)(keys + B);
     void* args[] = {&a0, &out_token, &V, &P, &keys, &cnt};
-    (void)hipLaunchKernel((const void*)vq::argmax_split_kernel, dim3((unsigned)(P * B)), dim3(vq::GR_NT), args, 0,
-                          (hipStream_t)stream);
+    (void)hipLaunchKernel(fn, dim3((unsigned)(P * B)), dim3(vq::GR_NT), args, 0, (hipStream_t)stream);
     return vq::status_of(hipGetLastError());
 }
