@@ -469,8 +469,8 @@ extern "C" int viper_hip_linear_bf16(const void* w_bf16, const void* x_bf16, voi
     if (lds > (size_t)vq::LDS_MAX || (size_t)K * 2 * 256 > (size_t)INT32_MAX) return VIPER_INVALID_ARGUMENT;
     // The dot kernel for one row and for the few whose LDS reads hide behind
     // the weights (M x K up to 4 x 2560: 121 us against 127 on the matrix
-    // cores; 3 rows of 4096: 163 against 157; 5 rows of 1024: 43.7 against 40.2).
-    if (M > 4 || (M > 1 && M * K > 10240)) {
+    // cores; 3 rows of 3840, N = 59702: 98 against 103; 3 rows of 4096: 163 against 157; 5 rows of 1024: 43.7 against 40.2).
+    if (M > 4 || (M > 1 && M * K >= 12288)) {
         const int tiles = (N + 15) / 16, waves = vq::HM_NTT / 64;
         int tpw = (tiles + 3 * vq::device_cus() - 1) / (3 * vq::device_cus());
         if (tpw < waves) tpw = waves;  // a tile for every wave

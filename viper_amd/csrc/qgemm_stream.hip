@@ -61,7 +61,15 @@ bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair) {
 // N = 10240 K = 4096 13.7 / 10.3; Q6 13.2 / 11.4; W8 N = 10240 K = 3072 16.3 /
 // 11.0; and where it holds them: Q4 N = 5120 K = 4096 6.4 / 6.8, K = 5120
 // 7.0 / 8.3, N = 10240 K = 3072 6.4 / 7.7).
-bool sg_takes(int qtype, int N, int K, bool pair) { return !rc_ok(qtype, K) || rc_capped(qtype, sg_rows(N, pair), K); }
+// Of those only K of one phase, or two of Q4 (K = 11776, N = 13696, M = 16
+// 40.8 / 30.6): serial phases cost more than rounds of workgroups (Q5, four
+// phases, K = 12800, N = 6400, M = 6 26.1 / 29.2; K = 12544, N = 7815, M = 3
+// 26.6 / 29.4).
+bool sg_takes(int qtype, int N, int K, bool pair) {
+    if (!rc_ok(qtype, K)) return true;
+    const int k_phase = qtype == VIPER_QTYPE_Q4_G64 ? (K + 127) / 128 * 64 : K;
+    return sg_one_phase(qtype, k_phase, RC_FRAG) && rc_capped(qtype, sg_rows(N, pair), K);
+}
 
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
               int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1, hipStream_t st) {

@@ -326,11 +326,13 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     // workgroup quantizing the bf16 rows of its own part of K, in one launch,
     // measured slower at every row count: down shape 3 / 8 / 16 rows 10.4 /
     // 12.6 / 15.9 us against 8.4 / 9.4 / 9.8 us.)
-    const bool split_ok = rc_k && b.w == nullptr && rc_split_blocks(qtype, N, K) > 0 && !rc_split_capped(qtype, N, K) && !one;
+    const bool takes = sg_takes(qtype, N, K, b.w != nullptr);
+    const bool split_ok = rc_k && b.w == nullptr && rc_split_blocks(qtype, N, K) > 0 &&
+                          !(takes && rc_split_capped(qtype, N, K)) && !one;
     // K or rows beyond the row-contiguous kernel: the streaming one, which also
     // quantizes up to 8 rows itself (Q4, M = 8, us, one launch / two: K = 3520,
     // N = 2560 6.1 / 7.0, N = 10240 9.8 / 10.6; K = 4096, N = 10240 9.9 / 10.6).
-    const bool sg = !split_ok && sg_takes(qtype, N, K, b.w != nullptr);
+    const bool sg = !split_ok && takes;
     // Q5/Q6/W8 (K = 2560, N = 10240, 5% outlier channels): 3 or 4 rows of one
     // matrix run faster on the multi-row dot kernel below (Q5 4 rows 7.86
     // against 8.10 us; W8 3 / 4 rows 7.47 / 7.77 against 8.9 / 9.17 us); 5-8
@@ -424,10 +426,11 @@ static int prequant_frag(int qtype, const void* w, const void* s, int senc, int 
     if (wsp != nullptr && misaligned(wsp, 16)) return VIPER_INVALID_ARGUMENT;
     const size_t need = b.w == nullptr ? frag_workspace_need(qtype, N, K, M) : 0;
     if (wsp != nullptr && need > 0 && wsp_bytes < need) return VIPER_INVALID_ARGUMENT;
-    const bool split = wsp != nullptr && need > 0 && !rc_split_capped(qtype, N, K);
+    const bool takes = sg_takes(qtype, N, K, b.w != nullptr);
+    const bool split = wsp != nullptr && need > 0 && !(takes && rc_split_capped(qtype, N, K));
     uint64_t* sp = split ? (uint64_t*)((uint8_t*)wsp + RC_CTL_BYTES) : nullptr;
     unsigned* sc = split ? (unsigned*)wsp : nullptr;
-    if (!split && sg_takes(qtype, N, K, b.w != nullptr))
+    if (!split && takes)
         return launch_sg(qtype, w, s, senc, N, K, xf, xsf, RC_FRAG, M, y, res, nullptr, b.w, b.s, b.y, (hipStream_t)stream);
     return launch_rc(qtype, w, s, senc, N, K, xf, xsf, RC_FRAG, M, y, res, nullptr, b.w, b.s, b.y,
                      (hipStream_t)stream, sp, sc);
