@@ -43,3 +43,42 @@ def test_head_rows_nonfinite(torch_dev):  # noqa: F811
     keep = np.ones((M, N), dtype=bool)
     keep[3], keep[:, 41] = False, False
     np.testing.assert_array_equal(y[keep], O.bf16_to_f32(clean)[keep])
+
+
+# Up to 8 tiles per workgroup, whose waves split the row segments of each: 256-element segments by one, two, four and
+# eight waves (fewer than waves, uneven, a short last one), a last workgroup with fewer tiles; the last shapes of one
+# round of workgroups (256 CUs) and the first of several.
+@pytest.mark.parametrize("M,N,K", [(5, 16, 264), (6, 33, 520), (16, 1000, 776), (16, 4096, 2048), (5, 4097, 2312),
+                                   (8, 8193, 1032), (3, 8500, 4104), (7, 12289, 520), (5, 16385, 264), (6, 32769, 264),
+                                   (5, 65520, 72), (5, 65521, 72)])
+def test_head_rows_shared_tiles(torch_dev, M, N, K):  # noqa: F811
+    test_head_rows(torch_dev, M, N, K)
+
+
+def test_head_few_weight_rows_spread(torch_dev):  # noqa: F811
+    # A sixteenth of the weight rows spreads over the CUs and takes well under the whole's time (measured 0.41; nine
+    # tiles to a workgroup's eight waves, whatever N, 0.79).
+    torch = torch_dev
+    M, K, reps = 8, 2560, 20
+    x = dev(torch, O.gen_act(M, K, 0x4EAF))
+    w = torch.full((reps, 16384, K), 0.01, dtype=torch.bfloat16, device="cuda").view(torch.int16)
+    y = torch.zeros((M, 16384), dtype=torch.int16, device="cuda")
+    us = {}
+    for N in (16384, 1024):
+        yn = y.view(-1)[:M * N].view(M, N)
+        best = 1e9
+        for _ in range(5):
+            torch.cuda.synchronize()
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            g = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(g):
+                for i in range(reps):
+                    assert va.linear_bf16(w[i, :N], x, yn).ok()
+            g.replay()
+            a.record()
+            g.replay()
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 1e3 / reps)
+        us[N] = best
+    assert us[1024] < 0.6 * us[16384], us

@@ -123,9 +123,8 @@ gemv_bf16_kernel(const uint16_t* __restrict__ w, const uint16_t* x, uint16_t* __
 // once; each wave keeps the next 8 KB segment (of the next tile, too) in
 // flight while it multiplies one.  Bound by the weight stream: 127 us for 2..6
 // rows, 129 for 8, 132 for 12 (850 MB, 6.5-6.7 TB/s; the dot kernel's one row
-// 117 us).  tpw tiles per workgroup: an odd number, about three workgroups per
-// CU (131072 x 4096: 157 us; 256 workgroups, whose first rows then lie 4 MB
-// apart and meet in the same memory channels, 178 us).
+// 117 us).  tpw tiles per workgroup; SHARE: a workgroup's few tiles go to 1 << lk
+// waves each, one tile a wave (hm_split).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -138,8 +137,9 @@ __host__ __device__ constexpr size_t hm_lds_bytes(int M, int K) {
     return (size_t)((K / 8 + HM_SC - 1) / HM_SC * HM_SC) * M * 16 + (size_t)(HM_NTT / 64) * 16 * HM_STR;
 }
 
+template <bool SHARE>
 __global__ void __launch_bounds__(HM_NTT)
-head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N, int K, int tpw, int gx) {
+head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N, int K, int tpw, int gx, int lk) {
     constexpr int W = HM_NTT / 64, RI = 64 / HM_SC;
     extern __shared__ __align__(16) u32x4 lx[];  // x as [chunk][M], zeros past the row; then the waves' buffers
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -150,6 +150,8 @@ head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N
     const int bid = ((int)blockIdx.x & 7) * gx + ((int)blockIdx.x >> 3);
     const int tend = min((bid + 1) * tpw, (N + 15) / 16);
     if (bid * tpw >= tend) return;
+    const int ks = SHARE ? 1 << lk : 1, s0 = SHARE ? wave & (ks - 1) : 0;  // segments s0, s0 + ks, ... of its tiles
+    const int t0 = bid * tpw + (SHARE ? wave >> lk : wave);
     const int nx = M * CPR;
     const auto xr = buf(x, (uint32_t)nx * 16);
     u32x4 xv[HM_XS];
@@ -165,9 +167,9 @@ head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N
     };
     const uint32_t rbytes = (uint32_t)K * 2;
     auto advance = [&](Cur& c) {
-        if (++c.s == NS) {
-            c.s = 0;
-            c.t += W;
+        if ((c.s += ks) >= NS) {
+            c.s = s0;
+            c.t += SHARE ? W >> lk : W;
         }
     };
     auto load = [&](Seg& S, const Cur& c) {
@@ -178,7 +180,7 @@ head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N
         for (int i = 0; i < 16 / RI; ++i)
             S.v[i] = bload16<AUX_NT>(wr, ch < CPR ? (i * RI + lane / HM_SC) * (int)rbytes + ch * 16 : OOB);
     };
-    Cur lc{bid * tpw + wave, 0}, cc = lc;
+    Cur lc{!SHARE || s0 < NS ? t0 : tend, s0}, cc = lc;
     Seg S0, S1;
     if (lc.t < tend) load(S0, lc);
     issue_fence();
@@ -195,6 +197,18 @@ head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N
 
     const int mr = min(l16, M - 1);  // columns past M repeat the last row and are not stored
     f32x4 a0 = {0.0f, 0.0f, 0.0f, 0.0f}, a1 = a0;
+    // the lane holds rows 4q .. 4q + 3 of a tile for activation row l16
+    auto store = [&](int t, const f32x4& v) {
+        const int n0 = t * 16 + 4 * q;
+        const uint32_t p0 = f2bf2(v[0], v[1]), p1 = f2bf2(v[2], v[3]);
+        if (l16 < M) {
+            uint16_t* o = y + (size_t)l16 * N + n0;
+            if (n0 < N) o[0] = (uint16_t)p0;
+            if (n0 + 1 < N) o[1] = (uint16_t)(p0 >> 16);
+            if (n0 + 2 < N) o[2] = (uint16_t)p1;
+            if (n0 + 3 < N) o[3] = (uint16_t)(p1 >> 16);
+        }
+    };
     auto compute = [&](const Seg& S, const Cur& c) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
         __builtin_amdgcn_wave_barrier();
@@ -215,17 +229,8 @@ head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N
             a1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w1), __builtin_bit_cast(bf16x8, x1),
                                                          a1, 0, 0, 0);
         }
-        if (c.s + 1 < NS) return;
-        // the lane holds rows 4q .. 4q + 3 of the tile for activation row l16
-        const int n0 = c.t * 16 + 4 * q;
-        const uint32_t p0 = f2bf2(a0[0] + a1[0], a0[1] + a1[1]), p1 = f2bf2(a0[2] + a1[2], a0[3] + a1[3]);
-        if (l16 < M) {
-            uint16_t* o = y + (size_t)l16 * N + n0;
-            if (n0 < N) o[0] = (uint16_t)p0;
-            if (n0 + 1 < N) o[1] = (uint16_t)(p0 >> 16);
-            if (n0 + 2 < N) o[2] = (uint16_t)p1;
-            if (n0 + 3 < N) o[3] = (uint16_t)(p1 >> 16);
-        }
+        if (SHARE || c.s + 1 < NS) return;
+        store(c.t, a0 + a1);
         a0 = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         a1 = a0;
     };
@@ -252,6 +257,17 @@ head_mfma_kernel(const uint16_t* w, const uint16_t* x, uint16_t* y, int M, int N
             compute(S1, cc);
             advance(cc);
         }
+    }
+    if constexpr (SHARE) {
+        // the waves of a tile meet in LDS, added in wave order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        *(f32x4*)(tb + lane * 16) = a0 + a1;
+        lds_barrier();
+        if (s0 != 0 || t0 >= tend) return;
+        f32x4 v = *(const f32x4*)(tb + lane * 16);
+        for (int u = 1; u < ks; ++u) v += *(const f32x4*)(tb + u * (16 * HM_STR) + lane * 16);
+        store(t0, v);
     }
 }
 
@@ -445,6 +461,43 @@ static lh_fn lh_pick(int mt, bool exact) {
     return exact ? lh_pick_mt<TS, true>(mt) : lh_pick_mt<TS, false>(mt);
 }
 
+// The matrix-core kernel's tiles per workgroup and (log2) waves per tile.  Up to
+// 16 tiles per CU: one round of workgroups, and where a workgroup has half as
+// many tiles as waves or fewer the waves split the rows of each, so that no
+// wave reads a row alone while others idle (8 rows of 2560, N = 1024 / 4096 /
+// 16384 18.6 / 19.1 / 22.3 us with nine tiles to eight waves -> 5.7 / 6.8 / 16.2;
+// 2 waves per tile at N = 4096 8.2, none 8.8; a second round of workgroups, 0.1
+// to 0.8 of the chip, is as long as the first: N = 40000 50 -> 36.5, N = 50257 52
+// -> 45).  Beyond, about three workgroups per CU in turn, each of an odd number
+// of tiles (131072 x 4096: 157 us; 256 workgroups, whose first rows then lie
+// 4 MB apart and meet in the same memory channels, 178 us; N = 65536, 4 rows of
+// 8192, 16 tiles each 205 us, 9 each 185).
+static void hm_split(int tiles, int segs, int& tpw, int& lk) {
+    const int cus = device_cus(), waves = HM_NTT / 64;
+    lk = 0;
+    if (tiles < 16 * cus) {
+        tpw = (tiles + cus - 1) / cus;
+        while (lk < 3 && tpw <= waves >> (lk + 1) && (1 << lk) < segs) ++lk;
+    } else {
+        tpw = (tiles + 3 * cus - 1) / (3 * cus);
+        tpw = (tpw < waves ? waves : tpw) | 1;
+    }
+}
+
+// Several rows on the matrix cores, or on the dot kernel?  The dot kernel for
+// the few rows whose LDS reads hide behind the weights (M x K up to 4 x 2560:
+// 121 us against 127; 3 rows of 4096: N = 65536 88 against 94, N = 131072 175
+// against 180; 4 rows of 3072 99 against 87 the other way, 5 rows of 1024: 43.7
+// against 40.2), for up to 4 rows also where N is small (3 rows of 4096, N = 300
+// / 1024 / 2560 5.3 / 5.9 / 8.4 us against 6.2 / 6.4 / 7.2), and for two rows of
+// a large head (8192, N = 16384 / 32000 / 65536 53.6 / 91 / 171 against 47 / 97 / 185).
+static bool hm_takes(int M, int N, int K) {
+    if (M > 4) return true;
+    if (M < 2 || N < 2048) return false;
+    if (M == 4) return K >= 3072;
+    return M * K > 12288 && (M == 3 || (N + 15) / 16 <= 4 * device_cus());
+}
+
 // Octets per thread of the split argmax.  Every workgroup's two atomics go to
 // the one or two cache lines that hold all rows' keys and counters and are
 // performed one after another there, ~15 ns each: with two octets per thread
@@ -467,19 +520,14 @@ extern "C" int viper_hip_linear_bf16(const void* w_bf16, const void* x_bf16, voi
         return VIPER_INVALID_ARGUMENT;
     const size_t lds = (size_t)M * K * 2;
     if (lds > (size_t)vq::LDS_MAX || (size_t)K * 2 * 256 > (size_t)INT32_MAX) return VIPER_INVALID_ARGUMENT;
-    // The dot kernel for one row and for the few whose LDS reads hide behind
-    // the weights (M x K up to 4 x 2560: 121 us against 127 on the matrix
-    // cores; 3 rows of 3840, N = 59702: 98 against 103; 3 rows of 4096: 163 against 157; 5 rows of 1024: 43.7 against 40.2).
-    if (M > 4 || (M > 1 && M * K >= 12288)) {
-        const int tiles = (N + 15) / 16, waves = vq::HM_NTT / 64;
-        int tpw = (tiles + 3 * vq::device_cus() - 1) / (3 * vq::device_cus());
-        if (tpw < waves) tpw = waves;  // a tile for every wave
-        tpw |= 1;
-        const int blocks = (tiles + tpw - 1) / tpw;
-        int gx = (blocks + 7) / 8;
-        void* args[] = {&w_bf16, &x_bf16, &y_bf16, &M, &N, &K, &tpw, &gx};
-        (void)hipLaunchKernel((const void*)vq::head_mfma_kernel, dim3((unsigned)(8 * gx)), dim3(vq::HM_NTT), args,
-                              vq::hm_lds_bytes(M, K), (hipStream_t)stream);
+    if (vq::hm_takes(M, N, K)) {
+        const int tiles = (N + 15) / 16;
+        int tpw = 0, lk = 0;
+        vq::hm_split(tiles, (K / 8 + vq::HM_SC - 1) / vq::HM_SC, tpw, lk);
+        int gx = ((tiles + tpw - 1) / tpw + 7) / 8;
+        const void* fn = lk ? (const void*)vq::head_mfma_kernel<true> : (const void*)vq::head_mfma_kernel<false>;
+        void* args[] = {&w_bf16, &x_bf16, &y_bf16, &M, &N, &K, &tpw, &gx, &lk};
+        (void)hipLaunchKernel(fn, dim3((unsigned)(8 * gx)), dim3(vq::HM_NTT), args, vq::hm_lds_bytes(M, K), (hipStream_t)stream);
         return vq::status_of(hipGetLastError());
     }
     const int cpr = K / 8;
