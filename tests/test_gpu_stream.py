@@ -79,3 +79,28 @@ def test_stream_pair_equals_chain(torch_dev, qtype, N, K, pro):  # noqa: F811
     torch.cuda.synchronize()
     for a, b in ((g1, g), (u1, u), (h, h2), (h1, h2)):
         np.testing.assert_array_equal(u16(a), u16(b))
+
+
+# Most slots per lane, one to three segments and staging rounds, and waves with no unit (few rows): the folded
+# prologues equal the producer's kernel followed by the int8 row.
+@pytest.mark.parametrize("qtype,N,K", [(O.Q6_G64, 1024, 10752), (O.Q6_G64, 3, 8256), (O.Q5_G64, 300, 12288),
+                                       (O.Q4_G64, 5, 20480), (O.Q4_G64, 2048, 12288), (O.W8_G32, 77, 8192)])
+@pytest.mark.parametrize("pro", [P.RMSNORM, P.SWIGLU])
+def test_stream_idle_waves_every_prologue(torch_dev, qtype, N, K, pro):  # noqa: F811
+    torch = torch_dev
+    G = O.group_size(qtype)
+    w = weights(torch, qtype, N, K, 0x57E00 + N, O.SCALE_BF16)[0]
+    a = dev(torch, O.gen_act(1, K, 0x57E10, outlier_frac=0.02))
+    b = dev(torch, bf16(1.0 + 0.1 * np.random.default_rng(3).standard_normal((1, K))))
+    res = dev(torch, O.gen_act(1, N, 5))
+    y, r = (torch.zeros((1, N), dtype=torch.int16, device="cuda") for _ in range(2))
+    xq = torch.zeros((1, K), dtype=torch.int8, device="cuda")
+    xs = torch.zeros((1, K // G), dtype=torch.float32, device="cuda")
+    assert va.linear_m1([w], pro, a, b.view(-1) if pro == P.RMSNORM else b, [y], eps=1e-6, residual=res).ok()
+    if pro == P.RMSNORM:
+        assert va.rmsnorm_quantize(a, b.view(-1), 1e-6, G, xq, xs).ok()
+    else:
+        assert va.swiglu_quantize(a, b, G, xq, xs).ok()
+    assert va.linear_m1([w], P.INT8, xq, xs, [r], residual=res).ok()
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(u16(y), u16(r))

@@ -37,8 +37,11 @@ namespace vq {
 // 256 and 1024 threads were within 5 % of 512 or slower over K = 512..16384
 // and N = 1024..28672 once two workgroups share a CU where they can.
 constexpr int ST_NTT = 512;  // threads per workgroup
-// Weight-issue delay, s_sleep units, as in qgemv_m1_kernel (0 and 2 equal; 6
-// 0.05-0.1 us slower: only one unit per wave goes out ahead of the quantize).
+// Weight-issue delay, s_sleep units, as in qgemv_m1_kernel.  Without one the
+// bf16 row's calls are 1-2 % faster (K = 5120, N = 1024 2.44 against 2.51 us) and
+// those with a second input 3-5 % slower, whose loads then queue behind the
+// weights (swiglu, Q4, K = 10240, N = 1024 4.13 against 4.05; K = 12288, N = 2560
+// 5.84 / 5.65); 5 is slower than 2 by 1 %.
 constexpr int ST_DELAY = 2;
 // Most chunk slots per lane (two units of more of Q5 / Q6 pass 256 registers).
 template <int F>
@@ -209,9 +212,12 @@ qgemv_stream_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16
             return bload16(xr, o * 16);
         }
     };
+    // (rounds past the row are not issued where the shape does not fix their number)
+    constexpr bool SKIP = CPL == ST_MAX<F>;
     u32x4 xv[XS], av[XS];
 #pragma unroll
     for (int i = 0; i < XS; ++i) {
+        if (SKIP && NTT * i >= noct) break;
         if constexpr (PRE) {
             const u32x2 q = bload8(xr, (tid + NTT * i) * 8);
             xv[i] = u32x4{q.x, q.y, 0u, 0u};
@@ -224,6 +230,7 @@ qgemv_stream_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < XS; ++i) {
+            if (SKIP && NTT * i >= noct) break;
             const int o = tid + NTT * i;
             if constexpr (PRE) xv[i].z = bload4(xsr, (o % OPC == 0) ? (o / OPG) * 4 : OOB);
             else av[i] = bload16(xsr, o * 16);
@@ -237,60 +244,58 @@ qgemv_stream_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16
     }
     stamp(1);
     if constexpr (ST_DELAY > 0) __builtin_amdgcn_s_sleep(ST_DELAY);
-    Cur lc{bid * upw + wave, 0}, cc = lc;
-    Tile T0, T1;
-    load(T0, lc);
-    issue_fence();
-
-    stamp(2);
-    // 2. quantize the activation into LDS
-    float inv = 0.0f;
-    if constexpr (PRO == PRO_RMSNORM) {
-        float ss = 0.0f;
+    // quantize the activation into LDS (the tiles in flight meanwhile)
+    auto stage = [&] {
+        stamp(2);
+        float inv = 0.0f;
+        if constexpr (PRO == PRO_RMSNORM) {
+            float ss = 0.0f;
+#pragma unroll
+            for (int i = 0; i < XS; ++i) {
+                if (SKIP && NTT * i >= noct) break;
+                const u32x4 v = xv[i];  // octets past the row are zero
+                const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float f = bf16f((wd[j >> 1] >> (16 * (j & 1))) & 0xffffu);
+                    ss = __builtin_fmaf(f, f, ss);
+                }
+            }
+            ss = team_sum<64>(ss);
+            if (lane == 0) lred[wave] = ss;
+            lds_barrier();
+            float t = 0.0f;
+#pragma unroll
+            for (int i = 0; i < W; ++i) t += lred[i];
+            inv = __builtin_amdgcn_rsqf(t / (float)K + epsv);
+        }
+        auto quant_store = [&](int o, const u32x4& v) { m1_quant_store<F, PRE>(o, v, noct, lxq, lcs); };
+        const int wave0 = tid & ~63;
 #pragma unroll
         for (int i = 0; i < XS; ++i) {
-            const u32x4 v = xv[i];  // octets past the row are zero
-            const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float f = bf16f((wd[j >> 1] >> (16 * (j & 1))) & 0xffffu);
-                ss = __builtin_fmaf(f, f, ss);
-            }
-        }
-        ss = team_sum<64>(ss);
-        if (lane == 0) lred[wave] = ss;
-        lds_barrier();
-        float t = 0.0f;
-#pragma unroll
-        for (int i = 0; i < W; ++i) t += lred[i];
-        inv = __builtin_amdgcn_rsqf(t / (float)K + epsv);
-    }
-    auto quant_store = [&](int o, const u32x4& v) { m1_quant_store<F, PRE>(o, v, noct, lxq, lcs); };
-    const int wave0 = tid & ~63;
-#pragma unroll
-    for (int i = 0; i < XS; ++i) {
-        if (wave0 + NTT * i < noct) {
-            const int o = tid + NTT * i;
-            if constexpr (TWO) {
-                const u32x4 v = m1_produce<PRO>(xv[i], av[i], inv);
-                if (PRO == PRO_RMSNORM && __builtin_expect(extra_out, 0) && blockIdx.x == 0) {
-                    uint16_t* xo = m1_xout();
-                    if (xo != nullptr && o < noct) *(u32x4*)(xo + (size_t)o * 8) = v;
+            if (wave0 + NTT * i < noct) {
+                const int o = tid + NTT * i;
+                if constexpr (TWO) {
+                    const u32x4 v = m1_produce<PRO>(xv[i], av[i], inv);
+                    if (PRO == PRO_RMSNORM && __builtin_expect(extra_out, 0) && blockIdx.x == 0) {
+                        uint16_t* xo = m1_xout();
+                        if (xo != nullptr && o < noct) *(u32x4*)(xo + (size_t)o * 8) = v;
+                    }
+                    quant_store(o, v);
+                } else {
+                    quant_store(o, xv[i]);
                 }
-                quant_store(o, v);
-            } else {
-                quant_store(o, xv[i]);
             }
         }
-    }
-    if constexpr (!TWO)
-        if (__builtin_expect(noct > XS * NTT, 0))
-            for (int o = tid + XS * NTT; (o & ~63) < noct; o += NTT) quant_store(o, load_x(o));
-    stamp(3);
-    lds_barrier();
-    stamp(4);
+        if constexpr (!TWO)
+            if (__builtin_expect(noct > XS * NTT, 0))
+                for (int o = tid + XS * NTT; (o & ~63) < noct; o += NTT) quant_store(o, load_x(o));
+        stamp(3);
+        lds_barrier();
+        stamp(4);
+    };
 
-    // 3. tiles in order
+    // 2. a tile's products
     float acc[R] = {};
     uint16_t gate = 0;
     auto compute = [&](Tile& T, const Cur& c) {
@@ -371,9 +376,23 @@ qgemv_stream_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16
             if (st) y[row0 + rl] = f2bf(res != nullptr ? v + bf16f(T.res) : v);
         }
     };
-    // (separate code for the last tile: a load that may or may not have been
-    // issued would make every wait behind it one for both)
-    if (cc.u < uend) {
+    // 3. tiles in order, one in flight while the other is summed.  Separate code
+    // for waves with no tile, and for the last: a load that may or may not
+    // have been issued would make every wait behind it one for both, and one
+    // out of range still takes the address unit's time (waves past the units
+    // issuing theirs: Q6, K = 10752, N = 1024 4.6 -> 3.7 us without; N = 1536
+    // 5.25 -> 4.9).  (A second tile ahead of the quantize: 5 % faster where no
+    // wave has a third and the tiles are small, 2-11 % slower else, as the
+    // activation then queues behind it.)  Every wave runs stage(), hence its
+    // barriers, exactly once.
+    Cur lc{bid * upw + wave, 0}, cc = lc;
+    Tile T0, T1;
+    if (lc.u >= uend) {
+        stage();
+    } else {
+        load(T0, lc);
+        issue_fence();
+        stage();
         for (;;) {
             advance(lc);
             if (lc.u >= uend) {
