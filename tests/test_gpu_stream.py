@@ -104,3 +104,21 @@ def test_stream_idle_waves_every_prologue(torch_dev, qtype, N, K, pro):  # noqa:
     assert va.linear_m1([w], P.INT8, xq, xs, [r], residual=res).ok()
     torch.cuda.synchronize()
     np.testing.assert_array_equal(u16(y), u16(r))
+
+
+# The pair equals the launch of both matrices also where single rows of the K take an exact tiling for some N.
+@pytest.mark.parametrize("qtype,N,K", [(O.Q4_G64, 2560, 5120), (O.Q4_G64, 4608, 5120), (O.Q4_G64, 1536, 6144),
+                                       (O.Q4_G64, 1280, 10240), (O.W8_G32, 2560, 5120), (O.Q5_G64, 1536, 20480)])
+@pytest.mark.parametrize("pro", [P.BF16, P.RMSNORM])
+def test_pair_equals_chain_over_tilings(torch_dev, qtype, N, K, pro):  # noqa: F811
+    torch = torch_dev
+    wg, wu = (weights(torch, qtype, N, K, 0x57F00 + i, O.SCALE_BF16)[0] for i in (0, 1))
+    x = dev(torch, O.gen_act(1, K, 0x57F10, outlier_frac=0.02))
+    gamma = dev(torch, bf16(1.0 + 0.1 * np.random.default_rng(4).standard_normal(K))) if pro == P.RMSNORM else None
+    h, g, u, g1, u1, g2, u2 = (torch.zeros((1, N), dtype=torch.int16, device="cuda") for _ in range(7))
+    assert va.linear_m1_swiglu(wg, wu, pro, x, gamma, h, eps=1e-6, gate_out=g, up_out=u).ok()
+    assert va.linear_m1([wg, wu], pro, x, gamma, [g1, u1], eps=1e-6).ok()
+    assert va.linear_m1([wg], pro, x, gamma, [g2], eps=1e-6).ok() and va.linear_m1([wu], pro, x, gamma, [u2], eps=1e-6).ok()
+    torch.cuda.synchronize()
+    for a, b in ((g, g1), (u, u1), (g, g2), (u, u2)):
+        np.testing.assert_array_equal(u16(a), u16(b))

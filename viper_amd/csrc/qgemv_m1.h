@@ -758,8 +758,9 @@ typedef void (*m1_fn)(const void*, const uint8_t*, const uint16_t*, uint16_t*, i
 // Launch shapes: (team size, workgroup size, chunk slots per lane).  One row:
 // the exact tilings of 80 and 96 chunks (K = 2560 and the reference engine's
 // 3072; the 384-thread one puts the engine's shorter matrices on exactly one
-// workgroup per CU), for W8 also 160 and 192 (the same K); every other K takes
-// the streaming kernel (qgemv_stream.h).  The longer ones serve 2-4 rows.
+// workgroup per CU), for W8 also 160 and 192 (the same K), and those of longer
+// rows where they spread over the CUs evenly (m1_tiled); every other call takes
+// the streaming kernel (qgemv_stream.h).  The longer ones also serve 2-4 rows.
 constexpr int M1_SHAPES[][3] = {{8, 128, 10}, {8, 192, 10}, {8, 320, 10}, {16, 256, 10}, {16, 640, 10},
                                 {32, 640, 10}, {64, 640, 10}, {16, 256, 5}, {16, 320, 5}, {16, 640, 5},
                                 {32, 640, 5}, {64, 640, 5}, {16, 256, 6}, {16, 320, 6}, {16, 384, 6},
@@ -769,13 +770,10 @@ constexpr int M1_SHAPES[][3] = {{8, 128, 10}, {8, 192, 10}, {8, 320, 10}, {16, 2
 // (m1_wide96 says when).
 constexpr int M1_WIDE96[3] = {16, 704, 6};
 
-// Rows of `cpr` chunks that one-row launches tile exactly here.  (At 160 and
-// more chunks of the nibble formats the streaming kernel is faster: K = 5120,
-// N = 4096 / 11008 4.19 / 7.64 -> 3.95 / 6.95 us, K = 10240, N = 2560 / 11008
-// 4.52 / 14.4 -> 4.37 / 11.6 us; at 80 and 96 it is equal or slower: K = 2560,
-// N = 2560 / 10240 2.70 / 4.5 against 2.83 / 4.5 us.)
+// Rows of `cpr` chunks with one-row exact tilings (m1_tiled says which calls
+// take them).
 __host__ __device__ constexpr bool m1_tiles(int f, int cpr) {
-    return cpr == 80 || cpr == 96 || (f == 8 && (cpr == 160 || cpr == 192));
+    return cpr == 80 || cpr == 96 || cpr == 640 || ((f == 4 || f == 8) && (cpr == 160 || cpr == 192 || cpr == 320));
 }
 
 template <int F, int SENC, int MODE, bool EXACT, int PRO, int MR>

@@ -163,8 +163,10 @@ bool m1_rows_ok(int qtype, int K, int M) {
 }
 
 bool m1_rows_exact(int qtype, int K, int M) {
-    const bool w8 = qtype == VIPER_QTYPE_W8_G32;
-    return m1_rows_ok(qtype, K, M) && m1_tiles(w8 ? 8 : 4, K / (w8 ? 16 : 32));
+    if (!m1_rows_ok(qtype, K, M)) return false;
+    const int ck = qtype == VIPER_QTYPE_W8_G32 ? 16 : 32, noct = M * (K / 8);
+    const M1Shape sh = m1_shape(K / ck, 1 << 14, device_cus(), (noct + M1_XS_MR - 1) / M1_XS_MR, noct, false, m1_mr(M));
+    return m1_exact(sh, K / ck, K / group_of(qtype));
 }
 
 bool m1_rows_pair(int qtype, int K, int M) {
@@ -210,7 +212,8 @@ static StShape st_shape(int qtype, int K, const int* n, int nouts, int cus) {
     // One workgroup per CU, or two where there are enough units for both and
     // the kernel's registers let two sit on a CU (at most 128 per lane): small
     // tiles from 10 units per CU on (Q4, K = 2048, N = 8192 / 20000: 3.72 / 6.5
-    // -> 3.49 / 5.55 us; N = 4096, 8 units: 2.88 -> 3.01 us), larger ones from
+    // -> 3.49 / 5.55 us; N = 4096, 8 units: 2.88 -> 3.01 us; Q5, K = 4096, N =
+    // 4608, 9 units: 4.35 -> 4.67), larger ones from
     // 24 on (K = 7168, N = 8192 / 3000: 7.55 / 4.15 -> 7.22 / 4.61 us).
     const bool two = s.cpl <= 2 ? u >= 10L * cus : s.cpl <= (wide ? 4 : 5) && u >= 24L * cus;
     const long wgs = (two ? 2L : 1L) * cus;
@@ -250,14 +253,52 @@ static size_t st_lds(int qtype, int K, const StShape& s) {
 
 static int st_kw(int K, const StShape& s) { return (int)((unsigned)(K / 32) | (unsigned)s.upw << 12 | (unsigned)s.gx << 22); }
 
-// One row of this K takes an exact tiling of qgemv_m1_kernel.
-static bool m1_tiled(int qtype, int K) {
+static bool folded_pro(int pro) { return pro == PRO_RMSNORM || pro == PRO_SWIGLU; }
+
+// The exact tiling one row of this K would run on (ntt 0: none).
+static M1Shape m1_one(int qtype, int K, int N, int cus, int pro, bool pair) {
     const bool w8 = qtype == VIPER_QTYPE_W8_G32;
-    return m1_tiles(w8 ? 8 : 4, K / (w8 ? 16 : 32));
+    const int cpr = K / (w8 ? 16 : 32), noct = K / 8;
+    M1Shape sh{0, 0, 0};
+    if (!m1_tiles(w8 ? 8 : qtype, cpr)) return sh;
+    // The folded prologues run fastest with one octet per thread (rmsnorm's
+    // row sum and swiglu's element work are then a single pass): take such a
+    // workgroup where a tiling allows it, even at a higher row load.
+    if (folded_pro(pro)) sh = m1_shape(cpr, N, cus, noct < 640 ? noct : 640, noct, pair);
+    if (sh.ntt == 0) sh = m1_shape(cpr, N, cus, 0, noct, pair);
+    return sh;
+}
+
+// One row takes the exact tiling `sh`, or the streaming kernel?  80 and 96
+// chunks (W8 also 160 and 192) always the tiling (K = 2560, N = 2560 / 10240
+// 2.70 / 4.5 us against 2.83 / 4.5).  Longer rows where the streaming kernel's
+// eight waves take a second and third turn and the tiling gives every CU one
+// workgroup with rows within 20 / 17 of the mean: Q4, 160 chunks, up to 20
+// rows per CU (K = 5120, N = 4608 / 5120 3.90 / 4.05 us against 4.23 / 4.36;
+// N = 6144, 40 rows on the fullest CU, 5.2 / 4.8), with the swiglu prologue,
+// one octet per thread there, uneven too (N = 3072 3.6 / 3.9); 192 chunks up
+// to 12 (K = 6144, N = 2560 3.3 / 3.5); 320 up to 10 (int8 row, K = 10240, N =
+// 2560 4.19 / 4.37; W8, K = 5120 3.90 / 4.03).  640 chunks, two segments or ten
+// slots there, for 5..10 rows (Q5, K = 20480, N = 1536 / 2560 7.4 / 9.1 against
+// 8.2 / 10.5; N = 3072 15.6 / 12.2; W8, K = 10240, N = 1536 4.77 / 4.9).
+// Only where no other launch's outputs have to have the same bits (alone): the
+// gate/up pair's equal those of viper_hip_qlinear_m1 from the same row, for
+// any N, and the streaming kernel sums a row in one order whatever N.
+static bool m1_tiled(int qtype, int K, const M1Shape& sh, int N, int cus, int pro, bool alone) {
+    if (sh.ntt == 0) return false;
+    const bool w8 = qtype == VIPER_QTYPE_W8_G32;
+    const int cpr = K / (w8 ? 16 : 32);
+    if (cpr <= 96 || (w8 && cpr <= 192)) return true;
+    if (!alone) return false;
+    const long rows = (N + cus - 1) / cus, load = m1_load(sh, N, cus);
+    if (cpr == 640) return rows > 4 && rows <= 10;
+    if (cpr == 192 && pro == PRO_SWIGLU) return false;  // (Q4, N = 3072 4.4 / 4.1)
+    if (rows <= 8 || rows > (cpr == 160 ? 20 : cpr == 192 ? 12 : 10)) return false;
+    return load * 17 <= rows * 20 || (cpr == 160 && pro == PRO_SWIGLU);
 }
 
 int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa, float eps, void* xout,
-              const M1Out* outs, int nouts, const void* res, int32_t* part, hipStream_t st, int M) {
+              const M1Out* outs, int nouts, const void* res, int32_t* part, hipStream_t st, int M, bool plain) {
     if (nouts < 1 || nouts > 3) return VIPER_INVALID_ARGUMENT;
     const int mr = m1_mr(M);
     if (mr > 1 && (nouts != 1 || (pro != PRO_BF16 && pro != PRO_INT8) || !m1_rows_ok(qtype, K, M)))
@@ -277,7 +318,9 @@ int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa
     size_t lds;
     int nb[3] = {0, 0, 0};
     int kg;  // the K slot: streaming launches pack more into it, exact tilings carry the grid size
-    if (mr == 1 && !m1_tiled(qtype, K)) {
+    M1Shape sh = mr == 1 ? m1_one(qtype, K, ntot, cus, pro, false) : M1Shape{0, 0, 0};
+    const bool alone = nouts == 1 && (plain || pro == PRO_INT8 || pro == PRO_SWIGLU);
+    if (mr == 1 && !m1_tiled(qtype, K, sh, ntot, cus, pro, alone)) {
         const int n[3] = {outs[0].n, nouts > 1 ? outs[1].n : 0, nouts > 2 ? outs[2].n : 0};
         const StShape ss = st_shape(qtype, K, n, nouts, cus);
         fn = st_kernel(qtype, ss, senc, part != nullptr ? M1_PART : M1_PLAIN, pro);
@@ -287,13 +330,7 @@ int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa
         lds = st_lds(qtype, K, ss);
         kg = st_kw(K, ss);
     } else {
-        // The folded prologues run fastest with one octet per thread (rmsnorm's
-        // row sum and swiglu's element work are then a single pass): take such
-        // a workgroup where a tiling allows it, even at a higher row load.
-        M1Shape sh{0, 0, 0};
-        if (folded) sh = m1_shape(K / ck, ntot, cus, noct < 640 ? noct : 640, noct);
-        if (sh.ntt == 0)
-            sh = m1_shape(K / ck, ntot, cus, mr > 1 ? (noct + M1_XS_MR - 1) / M1_XS_MR : 0, noct, false, mr);
+        if (mr > 1) sh = m1_shape(K / ck, ntot, cus, (noct + M1_XS_MR - 1) / M1_XS_MR, noct, false, mr);
         if (sh.ntt == 0) return VIPER_INVALID_ARGUMENT;
         if (!folded && nouts == 1 && mr == 1) sh = m1_q5_bf16(qtype, pro, ntot, cus, m1_wide96(qtype, K / ck, ntot, cus, sh));
         const int group = qtype == VIPER_QTYPE_W8_G32 ? 32 : 64;
@@ -337,8 +374,9 @@ int launch_m1_timeline(int qtype, int senc, int K, const void* x, const void* w,
     int nwg, threads, kg;  // as launch_m1
     unsigned grid;
     size_t lds;
-    if (m1_tiled(qtype, K)) {
-        const M1Shape sh = m1_q5_bf16(qtype, PRO_BF16, N, cus, m1_wide96(qtype, cpr, N, cus, m1_shape(cpr, N, cus, 0, K / 8)));
+    M1Shape sh = m1_one(qtype, K, N, cus, PRO_BF16, false);
+    if (m1_tiled(qtype, K, sh, N, cus, PRO_BF16, true)) {
+        sh = m1_q5_bf16(qtype, PRO_BF16, N, cus, m1_wide96(qtype, cpr, N, cus, sh));
         fn = m1_kernel(qtype, sh, senc, M1_TL, true, PRO_BF16);
         const int rows = sh.ntt / sh.ts;
         nwg = (N + rows - 1) / rows;
@@ -381,14 +419,13 @@ int launch_m1_swiglu(int qtype, int senc, int K, int pro, const void* x, const v
                      void* u_out, hipStream_t st) {
     if (pro != PRO_BF16 && pro != PRO_RMSNORM) return VIPER_INVALID_ARGUMENT;
     if (N >= M1_N_EXTRA) return VIPER_INVALID_ARGUMENT;  // n0's high bits carry flags
-    const int ck = qtype == VIPER_QTYPE_W8_G32 ? 16 : 32;
-    const int noct = K / 8;
     const int cus = device_cus();
     m1_fn fn;
     unsigned grid, threads;
     size_t lds;
     int kg;  // as in launch_m1
-    if (!m1_tiled(qtype, K)) {
+    const M1Shape sh = m1_one(qtype, K, N, cus, pro, true);
+    if (!m1_tiled(qtype, K, sh, N, cus, pro, false)) {
         const StShape ss = st_shape(qtype, K, &N, 1, cus);
         fn = st_kernel(qtype, ss, senc, M1_SWIGLU, pro);
         grid = (unsigned)ss.grid;
@@ -396,10 +433,6 @@ int launch_m1_swiglu(int qtype, int senc, int K, int pro, const void* x, const v
         lds = st_lds(qtype, K, ss);
         kg = st_kw(K, ss);
     } else {
-        M1Shape sh{0, 0, 0};
-        if (pro == PRO_RMSNORM) sh = m1_shape(K / ck, N, cus, noct < 640 ? noct : 640, noct, true);
-        if (sh.ntt == 0) sh = m1_shape(K / ck, N, cus, 0, noct, true);
-        if (sh.ntt == 0) return VIPER_INVALID_ARGUMENT;
         fn = m1_kernel(qtype, sh, senc, M1_SWIGLU, true, pro);
         const int rows = sh.ntt / sh.ts;
         grid = (unsigned)((N + rows / 2 - 1) / (rows / 2));

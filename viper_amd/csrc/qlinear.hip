@@ -602,7 +602,7 @@ extern "C" int viper_hip_qlinear_m1(int qtype, int scale_enc, int group, int K, 
     if ((prologue == VIPER_PROLOGUE_RMSNORM || prologue == VIPER_PROLOGUE_SWIGLU) && !vq::m1_folded_ok(qtype, K))
         return VIPER_INVALID_ARGUMENT;
     return vq::launch_m1(qtype, scale_enc, K, prologue, a, b, eps, norm_out, outs, n_out, residual_bf16, nullptr,
-                         (hipStream_t)stream);
+                         (hipStream_t)stream, 1, false);
 }
 
 extern "C" int viper_hip_qlinear_m1_swiglu(int qtype, int scale_enc, int group, int K, int prologue, const void* a,

@@ -93,9 +93,11 @@ struct M1Out {
 size_t lds_m1(int qtype, int K);
 bool m1_folded_ok(int qtype, int K);
 // M (1..4) activation rows: M > 1 needs one matrix, PRO_BF16 or PRO_INT8 and
-// m1_rows_ok (x, y, res and part hold M rows).
+// m1_rows_ok (x, y, res and part hold M rows).  plain: the row of a bf16 call
+// whose outputs no other entry point promises to match (m1_tiled).
 int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa, float eps, void* xout,
-              const M1Out* outs, int nouts, const void* res, int32_t* part, hipStream_t st, int M = 1);
+              const M1Out* outs, int nouts, const void* res, int32_t* part, hipStream_t st, int M = 1,
+              bool plain = true);
 bool m1_rows_ok(int qtype, int K, int M);
 bool m1_rows_exact(int qtype, int K, int M);
 // m1_rows_ok and the bf16 rows are staged two octets per thread (Q4, exact
