@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
+
 #include "qlinear_dev.h"
 
 namespace vq {
@@ -58,23 +60,30 @@ inline void launch(const void* fn, unsigned grid, unsigned block, size_t lds, hi
     (void)hipLaunchKernel(fn, dim3(grid), dim3(block), args, lds, st);
 }
 
-inline int device_cus() {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-        return 256;
-    return cus;
+// A positive property of the current device, asked for once per device (a
+// call's choice of kernel reads these several times: 0.1 us each time; the
+// values never change while the process lives).  `none` where there is no
+// device to ask.
+template <hipDeviceAttribute_t ATTR>
+inline int device_attribute(int none) {
+    constexpr int MAX_DEV = 64;
+    static std::atomic<int> known[MAX_DEV];  // 0: not asked yet
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return none;
+    if (dev >= 0 && dev < MAX_DEV && (v = known[dev].load(std::memory_order_relaxed)) > 0) return v;
+    if (hipDeviceGetAttribute(&v, ATTR, dev) != hipSuccess || v <= 0) return none;
+    if (dev >= 0 && dev < MAX_DEV) known[dev].store(v, std::memory_order_relaxed);
+    return v;
 }
+
+inline int device_cus() { return device_attribute<hipDeviceAttributeMultiprocessorCount>(256); }
 
 // LDS one workgroup may allocate on the current device (160 KB on gfx950).
 // Most launch choices keep to LDS_MAX; the bf16-quantizing matrix-core mode
 // stages a workgroup's activation fragments and uses the device's full budget.
 inline int device_lds_max() {
-    int dev = 0, lds = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return LDS_MAX;
-    if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || lds < LDS_MAX)
-        return LDS_MAX;
-    return lds;
+    const int lds = device_attribute<hipDeviceAttributeMaxSharedMemoryPerBlock>(LDS_MAX);
+    return lds < LDS_MAX ? LDS_MAX : lds;
 }
 
 // ---- launchers (one translation unit each)
