@@ -55,6 +55,8 @@
  *                                   block per row).
  *   viper_hip_qlinear_partials      no counterpart: the same kernels, also writing
  *                                   the exact per-group int32 dots for parity tests.
+ *   viper_hip_qlinear_route         no counterpart: which kernel a call of given
+ *                                   sizes runs (test and measurement).
  *   viper_hip_qlinear_timeline      no counterpart: the M = 1 GEMV with per-wave
  *                                   timestamps (measurement).
  *   viper_hip_qlinear_frag_timeline no counterpart: the M = 2..16 matrix-core GEMM
@@ -314,6 +316,25 @@ int viper_hip_check_bf16_rounding(unsigned long long* count, void* stream);
  * entries) receives the number of disagreements for amax bits
  * (exp_lo << 7) + i. */
 int viper_hip_check_quantizer(int exp_lo, int exp_hi, int32_t* counts, void* stream);
+
+/* Test and measurement use, no counterpart in the reference: the kernel that a
+ * call of these sizes runs on the current device (256 CUs without one), one of
+ * VIPER_ROUTE_*; -1 where the sizes or the input are invalid.  input: bf16 rows
+ * (viper_hip_qlinear, viper_hip_qlinear_fused2 for matrices = 2), int8 rows
+ * (the prequantized entry points) or fragments (with a workspace where the
+ * shape has one).  Reads nothing but the sizes; a call may still be refused
+ * for its other arguments. */
+#define VIPER_INPUT_BF16 0
+#define VIPER_INPUT_INT8 1
+#define VIPER_INPUT_FRAG 2
+#define VIPER_ROUTE_M1 0          /* one row: the M = 1 kernels */
+#define VIPER_ROUTE_ROWS 1        /* 2..4 rows on the M = 1 kernel's dot path */
+#define VIPER_ROUTE_RC_BF16 2     /* row-contiguous matrix-core kernel quantizing the rows itself */
+#define VIPER_ROUTE_STREAM_BF16 3 /* streaming matrix-core kernel quantizing the rows itself */
+#define VIPER_ROUTE_RC_SPLIT 4    /* the row-contiguous kernel's K split */
+#define VIPER_ROUTE_RC 5          /* the row-contiguous kernel on int8 rows */
+#define VIPER_ROUTE_STREAM 6      /* the streaming kernel on int8 rows */
+int viper_hip_qlinear_route(int qtype, int input, int N, int K, int M, int matrices);
 
 /* Measurement entry point, no counterpart in the reference: the M = 1 GEMV
  * of viper_hip_qlinear (any quantized format, bf16 x, launch shapes whose

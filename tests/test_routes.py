@@ -1,0 +1,29 @@
+"""Which kernel a call of given sizes runs (viper_hip_qlinear_route), at 256 CUs: sizes whose measured best kernel the
+rules must keep.  Needs no GPU; on one the same holds for the MI355X's 256 CUs."""
+import pytest
+
+import viper_amd as va
+
+Q4, Q5, Q6, W8 = 4, 5, 6, 8
+BF16, INT8, FRAG = 0, 1, 2
+M1, ROWS, RC_BF16, STREAM_BF16, RC_SPLIT, RC, STREAM = range(7)
+
+
+def route(qtype, rows, N, K, M, matrices=1):
+    return va.lib().viper_hip_qlinear_route(qtype, rows, N, K, M, matrices)
+
+
+@pytest.mark.parametrize("qtype,rows,N,K,M,matrices,want", [
+    (Q4, BF16, 10240, 2560, 1, 1, M1), (W8, INT8, 10240, 2560, 1, 2, M1), (Q4, BF16, 2560, 2560, 2, 1, ROWS),
+    (Q4, BF16, 10240, 2560, 8, 1, RC_BF16), (Q4, BF16, 10240, 2560, 16, 1, RC), (Q4, BF16, 2560, 10240, 16, 1, RC_SPLIT),
+    (Q4, FRAG, 2560, 10240, 16, 1, RC_SPLIT), (Q4, FRAG, 1024, 10240, 16, 2, RC), (Q5, BF16, 2560, 3520, 8, 1, STREAM_BF16),
+    (Q4, FRAG, 10240, 4096, 16, 1, STREAM), (W8, INT8, 10240, 3072, 16, 1, STREAM)])
+def test_route_basics(qtype, rows, N, K, M, matrices, want):
+    assert route(qtype, rows, N, K, M, matrices) == want
+
+
+@pytest.mark.parametrize("args", [(7, BF16, 64, 64, 2, 1), (Q4, 3, 64, 64, 2, 1), (Q4, BF16, 0, 64, 2, 1),
+                                  (Q4, BF16, 64, 96, 2, 1), (Q4, BF16, 64, 64, 17, 1), (Q4, BF16, 64, 64, 2, 3),
+                                  (Q4, FRAG, 64, 256, 1, 1), (Q4, FRAG, 64, 192, 2, 1), (Q4, BF16, 64, 0, 2, 1)])
+def test_route_invalid(args):
+    assert va.lib().viper_hip_qlinear_route(*args) == -1

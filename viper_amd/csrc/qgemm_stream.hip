@@ -37,15 +37,14 @@ static bool sg_launch(int qtype, long rows_total, int K, int M, int am, bool par
     return l.lds <= (size_t)device_lds_max();
 }
 
-// K fits the registers of one workgroup's waves.
-bool sg_one_phase(int qtype, int K, int am) {
-    const int F = qtype == VIPER_QTYPE_W8_G32 ? 8 : qtype;
-    return K / group_of(qtype) <= SG_W * 2 * sg_ni_max(F, am, false);
+// Phases over K: the groups one workgroup's waves hold in registers.
+int sg_phases(int qtype, int K, int am) {
+    const int F = qtype == VIPER_QTYPE_W8_G32 ? 8 : qtype, most = SG_W * 2 * sg_ni_max(F, am, false);
+    return (K / group_of(qtype) + most - 1) / most;
 }
 
-// RC_BF16: at most 8 rows (a workgroup's quantize of more costs more than the
-// quantize launch: K = 3520, N = 2560, Q4, M = 16: 8.3 us against 4.9 + 2.1),
-// one phase, every row's octet pairs in SG_XR rounds.
+// RC_BF16: at most 8 rows (the slots of the LDS copy), one phase, every row's
+// octet pairs in SG_XR rounds.
 bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair) {
     if (M > 8 || (long)M * K > (long)SG_XR * 64 * SG_W * 16) return false;
     SgLaunch l;
@@ -67,8 +66,7 @@ bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair) {
 // 26.6 / 29.4).
 bool sg_takes(int qtype, int N, int K, bool pair) {
     if (!rc_ok(qtype, K)) return true;
-    const int k_phase = qtype == VIPER_QTYPE_Q4_G64 ? (K + 127) / 128 * 64 : K;
-    return sg_one_phase(qtype, k_phase, RC_FRAG) && rc_capped(qtype, sg_rows(N, pair), K);
+    return sg_phases(qtype, K, RC_FRAG) <= (qtype == VIPER_QTYPE_Q4_G64 ? 2 : 1) && rc_capped(qtype, sg_rows(N, pair), K);
 }
 
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,

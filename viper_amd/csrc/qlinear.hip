@@ -290,6 +290,91 @@ static bool dot_rows(int qtype, int N, int K, int M, bool one) {
     return (per_cu > 32 && (K <= 2048 || (per_cu <= 48 && !rc_ok(qtype, K)))) || (w8 && K > 96 * 32 && !rc_ok(qtype, K) && per_cu <= 16);
 }
 
+// The kernel a call runs, from its sizes alone (the routes of include/viper_qlinear.h).
+enum Route {
+    R_M1 = VIPER_ROUTE_M1,
+    R_ROWS = VIPER_ROUTE_ROWS,
+    R_RC_BF16 = VIPER_ROUTE_RC_BF16,
+    R_SG_BF16 = VIPER_ROUTE_STREAM_BF16,
+    R_SPLIT = VIPER_ROUTE_RC_SPLIT,
+    R_RC = VIPER_ROUTE_RC,
+    R_SG = VIPER_ROUTE_STREAM,
+};
+
+// bf16 rows.  Few rows: every workgroup quantizes the rows itself, one launch
+// (the workspace stays required for M > 1 whichever kernel runs).  Two to four
+// rows of one matrix on the M = 1 kernel's dot path; 5..8 rows (and fused
+// pairs of 3..8) on the matrix cores with the quantize into LDS
+// (north-star shape: M = 5 6.63 us, 8 7.49 us against 8.21 / 8.25 us for
+// the next-best path; at M >= 10 the rows' quantize in every workgroup
+// costs more than the quantize launch).
+static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) {
+    if (fused_ok(qtype, M, K)) return R_M1;
+    const bool rc_k = M >= 2 && rc_ok(qtype, K);
+    // K or rows beyond the row-contiguous kernel: the streaming one, which also
+    // quantizes up to 8 rows itself (Q4, M = 8, us, one launch / two: K = 3520,
+    // N = 2560 6.1 / 7.0, N = 10240 9.8 / 10.6; K = 4096, N = 10240 9.9 / 10.6).
+    const bool one = sg_bf16_ok(qtype, N, K, M, pair);
+    const bool takes = sg_takes(qtype, N, K, pair);
+    const bool dot = !pair && dot_rows(qtype, N, K, M, one);
+    if (M == 2 && dot) return R_ROWS;
+    // Long K splits over workgroups in the two-launch path (down shape
+    // K = 10240, 4 rows 9.5 us against 10.3 us without the split).  (Every
+    // workgroup quantizing the bf16 rows of its own part of K, in one launch,
+    // measured slower at every row count: down shape 3 / 8 / 16 rows 10.4 /
+    // 12.6 / 15.9 us against 8.4 / 9.4 / 9.8 us.)
+    const bool split = rc_k && !pair && rc_split_blocks(qtype, N, K) > 0 && !(takes && rc_split_capped(qtype, N, K)) && !one;
+    // Q5/Q6/W8 (K = 2560, N = 10240, 5% outlier channels): 3 or 4 rows of one
+    // matrix run faster on the multi-row dot kernel below (Q5 4 rows 7.86
+    // against 8.10 us; W8 3 / 4 rows 7.47 / 7.77 against 8.9 / 9.17 us); 5-8
+    // rows of every format stay on the one-launch path.
+    // (Q4 rows staged two octets per thread also past that size: down shape
+    // K = 10240, 4 rows 8.4 us against 9.0-9.1 us for two launches with the K
+    // split)
+    const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M));
+    // With the rows staged two octets per thread (64-groups), the row-contiguous
+    // kernel's one-launch path also wins for Q4 at 3-4 rows (5.45 / 5.74 against
+    // 5.6 / 5.9 us on the dot kernel) and 9-10 rows (6.76 / 7.00 against 7.27 us
+    // in two launches; 12 and 16 rows stay two launches: 7.5 / 8.2 against 7.3
+    // us), and for Q5 / Q6 at 8 rows (7.90 / 8.22 against 8.37 / 8.58 us).  W8
+    // keeps 3-4 rows on the dot kernel and 5-8 here.
+    const bool q4 = qtype == VIPER_QTYPE_Q4_G64;
+    const int bf_max = q4 && !pair ? 10 : 8;
+    const bool rc_bf16 = rc_k && !takes && M <= bf_max && !split && rc_bf16_ok(qtype, N, K, M, pair);
+    if (rc_bf16 && (M > 4 || !rows_ok || q4)) return R_RC_BF16;
+    // (3 or 4 rows here also where the LDS copy does not fit: while every
+    // workgroup's share of the rows' quantize stays small; down shape
+    // K = 10240: 3 rows 8.8 us against about 9.5 us for two launches with the K
+    // split)
+    if (rows_ok) return R_ROWS;
+    if (split) return R_SPLIT;
+    if (takes && one && !part) return R_SG_BF16;
+    return takes ? R_SG : R_RC;
+}
+
+// int8 rows in the layout of viper_hip_quantize_act.
+static Route prequant_route(int qtype, int N, int K, int M, bool pair) {
+    if (fused_ok(qtype, M, K)) return R_M1;
+    const bool one = sg_phases(qtype, K, RC_NAT) == 1;
+    // (a K of whole group quads has no workgroup quantize here: on the matrix
+    // cores it is faster at many rows too, Q4 K = 2048, 2 rows, N = 10240 6.3 / 5.1)
+    if (!pair && dot_rows(qtype, N, K, M, one) && (m1_rows_exact(qtype, K, M) || !one || !rc_ok(qtype, K))) return R_ROWS;
+    return M < 2 || sg_takes(qtype, N, K, pair) ? R_SG : R_RC;
+}
+
+// int8 fragments; ws: with a workspace the K split may use.
+static Route frag_route(int qtype, int N, int K, int M, bool pair, bool ws) {
+    const bool takes = sg_takes(qtype, N, K, pair);
+    if (ws && !pair && frag_workspace_need(qtype, N, K, M) > 0 && !(takes && rc_split_capped(qtype, N, K))) return R_SPLIT;
+    return takes ? R_SG : R_RC;
+}
+
+// The rows' limit of a call that neither the M = 1 kernels nor the
+// row-contiguous kernel take: one row, or K of an odd number of groups.
+static bool rows_refused(int qtype, int M, int K) {
+    return (M < 2 || (K / group_of(qtype)) % 2 != 0) && lds_pre(qtype, M, K) > (size_t)LDS_MAX;
+}
+
 static int qlinear_common(int qtype, const void* w, const void* s, int senc, int group, int N,
                           int K, const void* x, int M, void* y, const void* res, void* wsp,
                           size_t wsp_bytes, int32_t* part, void* stream, Second b = Second()) {
@@ -301,81 +386,34 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     rc = validate_second(b, qtype, senc, group, N, K, M, res, part);
     if (rc != VIPER_OK) return rc;
     hipStream_t st = (hipStream_t)stream;
+    const bool pair = b.w != nullptr;
     if (fused_ok(qtype, M, K)) {
         const M1Out outs[2] = {{w, s, y, N}, {b.w, b.s, b.y, N}};
-        return launch_m1(qtype, senc, K, PRO_BF16, x, nullptr, 0.0f, nullptr, outs, b.w ? 2 : 1, res, part, st);
+        return launch_m1(qtype, senc, K, PRO_BF16, x, nullptr, 0.0f, nullptr, outs, pair ? 2 : 1, res, part, st);
     }
     const size_t need = workspace_need(qtype, N, K, M);
     if (wsp == nullptr || wsp_bytes < need || misaligned(wsp, 16)) return VIPER_INVALID_ARGUMENT;
-    // Few rows: every workgroup quantizes the rows itself, one launch (the
-    // workspace stays required for M > 1 whichever kernel runs).  Two to four
-    // rows of one matrix on the M = 1 kernel's dot path; 5..8 rows (and fused
-    // pairs of 3..8) on the matrix cores with the quantize into LDS
-    // (north-star shape: M = 5 6.63 us, 8 7.49 us against 8.21 / 8.25 us for
-    // the next-best path; at M >= 10 the rows' quantize in every workgroup
-    // costs more than the quantize launch).
-    const bool rc_k = M >= 2 && rc_ok(qtype, K);
-    const bool one = sg_bf16_ok(qtype, N, K, M, b.w != nullptr);
-    const bool dot = b.w == nullptr && dot_rows(qtype, N, K, M, one);
-    if (M == 2 && dot) {
-        const M1Out outs[1] = {{w, s, y, N}};
-        return launch_m1(qtype, senc, K, PRO_BF16, x, nullptr, 0.0f, nullptr, outs, 1, res, part, st, M);
-    }
-    // Long K splits over workgroups in the two-launch path (down shape
-    // K = 10240, 4 rows 9.5 us against 10.3 us without the split).  (Every
-    // workgroup quantizing the bf16 rows of its own part of K, in one launch,
-    // measured slower at every row count: down shape 3 / 8 / 16 rows 10.4 /
-    // 12.6 / 15.9 us against 8.4 / 9.4 / 9.8 us.)
-    const bool takes = sg_takes(qtype, N, K, b.w != nullptr);
-    const bool split_ok = rc_k && b.w == nullptr && rc_split_blocks(qtype, N, K) > 0 &&
-                          !(takes && rc_split_capped(qtype, N, K)) && !one;
-    // K or rows beyond the row-contiguous kernel: the streaming one, which also
-    // quantizes up to 8 rows itself (Q4, M = 8, us, one launch / two: K = 3520,
-    // N = 2560 6.1 / 7.0, N = 10240 9.8 / 10.6; K = 4096, N = 10240 9.9 / 10.6).
-    const bool sg = !split_ok && takes;
-    // Q5/Q6/W8 (K = 2560, N = 10240, 5% outlier channels): 3 or 4 rows of one
-    // matrix run faster on the multi-row dot kernel below (Q5 4 rows 7.86
-    // against 8.10 us; W8 3 / 4 rows 7.47 / 7.77 against 8.9 / 9.17 us); 5-8
-    // rows of every format stay on the one-launch path.
-    // (Q4 rows staged two octets per thread also past that size: down shape
-    // K = 10240, 4 rows 8.4 us against 9.0-9.1 us for two launches with the K
-    // split)
-    const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M));
-    // With the rows staged two octets per thread (64-groups), the one-launch
-    // path also wins for Q4 at 3-4 rows (5.45 / 5.74 against 5.6 / 5.9 us on the
-    // dot kernel) and 9-10 rows (6.76 / 7.00 against 7.27 us in two launches;
-    // 12 and 16 rows stay two launches: 7.5 / 8.2 against 7.3 us), and for
-    // Q5 / Q6 at 8 rows (7.90 / 8.22 against 8.37 / 8.58 us).  W8 keeps 3-4
-    // rows on the dot kernel and 5-8 here.
-    const bool q4 = qtype == VIPER_QTYPE_Q4_G64;
-    const int bf_max = q4 && b.w == nullptr ? 10 : 8;
-    const bool bf_ok = rc_k && !sg && M <= bf_max && !split_ok && rc_bf16_ok(qtype, N, K, M, b.w != nullptr);
-    if (bf_ok && (M > 4 || !rows_ok || q4))
+    const Route route = linear_route(qtype, N, K, M, pair, part != nullptr);
+    if (route == R_RC_BF16)
         return launch_rc(qtype, w, s, senc, N, K, x, nullptr, RC_BF16, M, y, res, part, b.w, b.s, b.y, st);
-    // (3 or 4 rows here also where the LDS copy does not fit: while every
-    // workgroup's share of the rows' quantize stays small; down shape
-    // K = 10240: 3 rows 8.8 us against about 9.5 us for two launches with the K
-    // split)
-    if (rows_ok) {
+    if (route == R_ROWS) {
         const M1Out outs[1] = {{w, s, y, N}};
         return launch_m1(qtype, senc, K, PRO_BF16, x, nullptr, 0.0f, nullptr, outs, 1, res, part, st, M);
     }
-    // one row or an odd number of groups: K has a limit
-    if ((M < 2 || (K / group_of(qtype)) % 2 != 0) && lds_pre(qtype, M, K) > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
-    if (sg && part == nullptr && one)
+    if (rows_refused(qtype, M, K)) return VIPER_INVALID_ARGUMENT;
+    if (route == R_SG_BF16)
         return launch_sg(qtype, w, s, senc, N, K, x, nullptr, RC_BF16, M, y, res, nullptr, b.w, b.s, b.y, st);
     const WsLayout lay = workspace_layout(qtype, N, K, M);
-    if (split_ok && lay.blocks == 0) return VIPER_INTERNAL;
+    if (route == R_SPLIT && lay.blocks == 0) return VIPER_INTERNAL;
     uint8_t* xq = (uint8_t*)wsp + lay.xq;
     float* xs = (float*)((uint8_t*)wsp + lay.xs);
     // long K on the matrix cores: the K split (control words and counters at
     // the workspace's start, then the records of part sums)
-    const bool split = split_ok;
-    uint64_t* sp = split ? (uint64_t*)((uint8_t*)wsp + lay.sp) : nullptr;
-    unsigned* sc = split ? (unsigned*)wsp : nullptr;
+    uint64_t* sp = route == R_SPLIT ? (uint64_t*)((uint8_t*)wsp + lay.sp) : nullptr;
+    unsigned* sc = route == R_SPLIT ? (unsigned*)wsp : nullptr;
     rc = launch_quantize(group, x, M, K, xq, xs, true, st);
     if (rc != VIPER_OK) return rc;
-    if (sg || !rc_k)
+    if (route == R_SG)
         return launch_sg(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st);
     return launch_rc(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st, sp, sc);
 }
@@ -391,19 +429,13 @@ static int prequant_common(int qtype, const void* w, const void* s, int senc, in
     rc = validate_second(b, qtype, senc, group, N, K, M, res, nullptr);
     if (rc != VIPER_OK) return rc;
     hipStream_t st = (hipStream_t)stream;
-    if (fused_ok(qtype, M, K)) {
+    const Route route = prequant_route(qtype, N, K, M, b.w != nullptr);
+    if (route == R_M1 || route == R_ROWS) {
         const M1Out outs[2] = {{w, s, y, N}, {b.w, b.s, b.y, N}};
-        return launch_m1(qtype, senc, K, PRO_INT8, xq, xs, 0.0f, nullptr, outs, b.w ? 2 : 1, res, nullptr, st);
+        return launch_m1(qtype, senc, K, PRO_INT8, xq, xs, 0.0f, nullptr, outs, b.w ? 2 : 1, res, nullptr, st, M);
     }
-    // (a K of whole group quads has no workgroup quantize here: on the matrix
-    // cores it is faster at many rows too, Q4 K = 2048, 2 rows, N = 10240 6.3 / 5.1)
-    if (b.w == nullptr && dot_rows(qtype, N, K, M, sg_one_phase(qtype, K, RC_NAT)) &&
-        (m1_rows_exact(qtype, K, M) || !sg_one_phase(qtype, K, RC_NAT) || !rc_ok(qtype, K))) {
-        const M1Out outs[1] = {{w, s, y, N}};
-        return launch_m1(qtype, senc, K, PRO_INT8, xq, xs, 0.0f, nullptr, outs, 1, res, nullptr, st, M);
-    }
-    if ((M < 2 || (K / group) % 2 != 0) && lds_pre(qtype, M, K) > (size_t)LDS_MAX) return VIPER_INVALID_ARGUMENT;
-    if (M < 2 || sg_takes(qtype, N, K, b.w != nullptr))
+    if (rows_refused(qtype, M, K)) return VIPER_INVALID_ARGUMENT;
+    if (route == R_SG)
         return launch_sg(qtype, w, s, senc, N, K, xq, xs, RC_NAT, M, y, res, nullptr, b.w, b.s, b.y, st);
     return launch_rc(qtype, w, s, senc, N, K, xq, xs, RC_NAT, M, y, res, nullptr, b.w, b.s, b.y, st);
 }
@@ -426,12 +458,11 @@ static int prequant_frag(int qtype, const void* w, const void* s, int senc, int 
     if (wsp != nullptr && misaligned(wsp, 16)) return VIPER_INVALID_ARGUMENT;
     const size_t need = b.w == nullptr ? frag_workspace_need(qtype, N, K, M) : 0;
     if (wsp != nullptr && need > 0 && wsp_bytes < need) return VIPER_INVALID_ARGUMENT;
-    const bool takes = sg_takes(qtype, N, K, b.w != nullptr);
-    const bool split = wsp != nullptr && need > 0 && !(takes && rc_split_capped(qtype, N, K));
-    uint64_t* sp = split ? (uint64_t*)((uint8_t*)wsp + RC_CTL_BYTES) : nullptr;
-    unsigned* sc = split ? (unsigned*)wsp : nullptr;
-    if (!split && takes)
+    const Route route = frag_route(qtype, N, K, M, b.w != nullptr, wsp != nullptr);
+    if (route == R_SG)
         return launch_sg(qtype, w, s, senc, N, K, xf, xsf, RC_FRAG, M, y, res, nullptr, b.w, b.s, b.y, (hipStream_t)stream);
+    uint64_t* sp = route == R_SPLIT ? (uint64_t*)((uint8_t*)wsp + RC_CTL_BYTES) : nullptr;
+    unsigned* sc = route == R_SPLIT ? (unsigned*)wsp : nullptr;
     return launch_rc(qtype, w, s, senc, N, K, xf, xsf, RC_FRAG, M, y, res, nullptr, b.w, b.s, b.y,
                      (hipStream_t)stream, sp, sc);
 }
@@ -496,6 +527,20 @@ extern "C" int viper_hip_qlinear_partials(int qtype, const void* w_packed, const
     if (partials == nullptr) return VIPER_INVALID_ARGUMENT;
     return vq::qlinear_common(qtype, w_packed, w_scales, scale_enc, group, N, K, x_bf16, M, y_bf16,
                               residual_bf16, workspace, workspace_bytes, partials, stream);
+}
+
+extern "C" int viper_hip_qlinear_route(int qtype, int input, int N, int K, int M, int matrices) {
+    const int G = vq::group_of(qtype);
+    if (G == 0 || N <= 0 || K <= 0 || M <= 0 || M > VIPER_QLINEAR_MAX_M || K > VIPER_QLINEAR_MAX_K || K % G != 0 ||
+        matrices < 1 || matrices > 2)
+        return -1;
+    const bool pair = matrices == 2;
+    switch (input) {
+        case VIPER_INPUT_BF16: return vq::linear_route(qtype, N, K, M, pair, false);
+        case VIPER_INPUT_INT8: return vq::prequant_route(qtype, N, K, M, pair);
+        case VIPER_INPUT_FRAG: return M < 2 || !vq::rc_ok(qtype, K) ? -1 : (int)vq::frag_route(qtype, N, K, M, pair, true);
+        default: return -1;
+    }
 }
 
 extern "C" int viper_hip_quantize_act(int group, const void* x_bf16, int M, int K, void* xq,

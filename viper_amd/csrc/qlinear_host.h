@@ -82,7 +82,7 @@ inline int device_cus() { return device_attribute<hipDeviceAttributeMultiprocess
 // Most launch choices keep to LDS_MAX; the bf16-quantizing matrix-core mode
 // stages a workgroup's activation fragments and uses the device's full budget.
 inline int device_lds_max() {
-    const int lds = device_attribute<hipDeviceAttributeMaxSharedMemoryPerBlock>(LDS_MAX);
+    const int lds = device_attribute<hipDeviceAttributeMaxSharedMemoryPerBlock>(160 * 1024);
     return lds < LDS_MAX ? LDS_MAX : lds;
 }
 
@@ -173,7 +173,7 @@ int launch_rc_timeline(int qtype, const void* w, const void* s, int senc, int N,
 // M = 1..16, any K (qgemm_stream.hip): persistent workgroups, the activation
 // operands in registers.  am as for launch_rc; part only with RC_FRAG.
 bool sg_takes(int qtype, int N, int K, bool pair);
-bool sg_one_phase(int qtype, int K, int am);
+int sg_phases(int qtype, int K, int am);  // over K: what one workgroup's waves hold in registers
 bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair);
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
               int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1, hipStream_t st);

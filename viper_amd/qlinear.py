@@ -144,6 +144,7 @@ _SYMBOLS = (
     "viper_hip_qlinear_frag_workspace_bytes",
     "viper_hip_qlinear_fused2_prequantized_frag",
     "viper_hip_qlinear_frag_timeline",
+    "viper_hip_qlinear_route",
 )
 
 
@@ -203,6 +204,8 @@ def lib():
     L.viper_hip_qlinear_frag_timeline.argtypes = [i32, vp, vp, i32, i32, i32, i32, vp, vp, i32, vp, vp, sz, vp, vp,
                                                   vp, sz, vp]
     L.viper_hip_qlinear_frag_timeline.restype = i32
+    L.viper_hip_qlinear_route.argtypes = [i32, i32, i32, i32, i32, i32]
+    L.viper_hip_qlinear_route.restype = i32
     L.viper_hip_qlinear_fused2.argtypes = [i32, vp, vp, vp, vp, i32, i32, i32, i32, vp, i32, vp, vp, vp, sz, vp]
     L.viper_hip_qlinear_fused2.restype = i32
     L.viper_hip_qlinear_fused2_prequantized.argtypes = [i32, vp, vp, vp, vp, i32, i32, i32, i32, vp, vp, i32,
