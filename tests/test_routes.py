@@ -27,3 +27,10 @@ def test_route_basics(qtype, rows, N, K, M, matrices, want):
                                   (Q4, FRAG, 64, 256, 1, 1), (Q4, FRAG, 64, 192, 2, 1), (Q4, BF16, 64, 0, 2, 1)])
 def test_route_invalid(args):
     assert va.lib().viper_hip_qlinear_route(*args) == -1
+
+
+# Q4, long K: the K split unless one launch serves a K of one phase (7 and 8 rows of K = 6144 are past its LDS).
+@pytest.mark.parametrize("N,K,M,want", [(3072, 5376, 8, RC_SPLIT), (3072, 6144, 7, RC_SPLIT), (3072, 6144, 8, RC_SPLIT),
+                                        (3072, 6144, 6, RC_BF16), (3072, 5376, 7, RC_BF16), (3072, 6144, 16, RC_SPLIT)])
+def test_route_k_split(N, K, M, want):
+    assert route(Q4, BF16, N, K, M) == want

@@ -318,20 +318,6 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     const bool takes = sg_takes(qtype, N, K, pair);
     const bool dot = !pair && dot_rows(qtype, N, K, M, one);
     if (M == 2 && dot) return R_ROWS;
-    // Long K splits over workgroups in the two-launch path (down shape
-    // K = 10240, 4 rows 9.5 us against 10.3 us without the split).  (Every
-    // workgroup quantizing the bf16 rows of its own part of K, in one launch,
-    // measured slower at every row count: down shape 3 / 8 / 16 rows 10.4 /
-    // 12.6 / 15.9 us against 8.4 / 9.4 / 9.8 us.)
-    const bool split = rc_k && !pair && rc_split_blocks(qtype, N, K) > 0 && !(takes && rc_split_capped(qtype, N, K)) && !one;
-    // Q5/Q6/W8 (K = 2560, N = 10240, 5% outlier channels): 3 or 4 rows of one
-    // matrix run faster on the multi-row dot kernel below (Q5 4 rows 7.86
-    // against 8.10 us; W8 3 / 4 rows 7.47 / 7.77 against 8.9 / 9.17 us); 5-8
-    // rows of every format stay on the one-launch path.
-    // (Q4 rows staged two octets per thread also past that size: down shape
-    // K = 10240, 4 rows 8.4 us against 9.0-9.1 us for two launches with the K
-    // split)
-    const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M));
     // With the rows staged two octets per thread (64-groups), the row-contiguous
     // kernel's one-launch path also wins for Q4 at 3-4 rows (5.45 / 5.74 against
     // 5.6 / 5.9 us on the dot kernel) and 9-10 rows (6.76 / 7.00 against 7.27 us
@@ -340,8 +326,25 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // keeps 3-4 rows on the dot kernel and 5-8 here.
     const bool q4 = qtype == VIPER_QTYPE_Q4_G64;
     const int bf_max = q4 && !pair ? 10 : 8;
-    const bool rc_bf16 = rc_k && !takes && M <= bf_max && !split && rc_bf16_ok(qtype, N, K, M, pair);
-    if (rc_bf16 && (M > 4 || !rows_ok || q4)) return R_RC_BF16;
+    const bool rc_bf16 = rc_k && !takes && M <= bf_max && rc_bf16_ok(qtype, N, K, M, pair);
+    // Long K splits over workgroups in the two-launch path (down shape
+    // K = 10240, 4 rows 9.5 us against 10.3 us without the split), unless one
+    // launch serves a K of one phase (Q4, 6 rows, K = 6144, N = 3072 6.8 us
+    // against 8.5; 7 and 8 rows have none there: 8.5 against 9.2 on the segment
+    // loop).  (Every workgroup quantizing the bf16 rows of its own part of K,
+    // in one launch, measured slower at every row count: down shape 3 / 8 / 16
+    // rows 10.4 / 12.6 / 15.9 us against 8.4 / 9.4 / 9.8 us.)
+    const bool split = rc_k && !pair && rc_split_blocks(qtype, N, K) > 0 && !(takes && rc_split_capped(qtype, N, K)) &&
+                       !(one && (takes || rc_bf16));
+    // Q5/Q6/W8 (K = 2560, N = 10240, 5% outlier channels): 3 or 4 rows of one
+    // matrix run faster on the multi-row dot kernel below (Q5 4 rows 7.86
+    // against 8.10 us; W8 3 / 4 rows 7.47 / 7.77 against 8.9 / 9.17 us); 5-8
+    // rows of every format stay on the one-launch path.
+    // (Q4 rows staged two octets per thread also past that size: down shape
+    // K = 10240, 4 rows 8.4 us against 9.0-9.1 us for two launches with the K
+    // split)
+    const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M));
+    if (rc_bf16 && !split && (M > 4 || !rows_ok || q4)) return R_RC_BF16;
     // (3 or 4 rows here also where the LDS copy does not fit: while every
     // workgroup's share of the rows' quantize stays small; down shape
     // K = 10240: 3 rows 8.8 us against about 9.5 us for two launches with the K
