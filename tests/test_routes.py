@@ -34,3 +34,12 @@ def test_route_invalid(args):
                                         (3072, 6144, 6, RC_BF16), (3072, 5376, 7, RC_BF16), (3072, 6144, 16, RC_SPLIT)])
 def test_route_k_split(N, K, M, want):
     assert route(Q4, BF16, N, K, M) == want
+
+
+# Q4, K of two phases: few rows quantized by every workgroup of the row-contiguous kernel while its rounds are few, then
+# the streaming kernel's two launches; the dots up to 40 rows per CU.  A pair's two rows up to two rounds.
+@pytest.mark.parametrize("qtype,N,K,M,matrices,want", [
+    (Q4, 10240, 7168, 3, 1, RC_BF16), (Q4, 8192, 7168, 4, 1, RC_BF16), (Q4, 10240, 7168, 5, 1, STREAM),
+    (Q4, 16384, 7168, 4, 1, STREAM), (Q4, 4352, 9216, 3, 1, ROWS), (Q5, 24576, 2048, 2, 2, RC)])
+def test_route_two_phases(qtype, N, K, M, matrices, want):
+    assert route(qtype, BF16, N, K, M, matrices) == want

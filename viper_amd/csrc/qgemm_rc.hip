@@ -150,6 +150,13 @@ bool rc_capped(int qtype, long rows_total, int K) {
     return bounded && rows_total > 8L * sh.rb * device_cus();
 }
 
+int rc_rounds(int qtype, long rows_total, int K, int* rows) {
+    const RcShape sh = rc_launch_shape(qtype, (int)(rows_total < 1 << 28 ? rows_total : 1 << 28), K);
+    const long per = 8L * sh.rb * device_cus();
+    *rows = 8 * sh.rb;
+    return sh.w == 4 ? 1 : (int)((rows_total + per - 1) / per);  // (4 waves: several workgroups share a CU)
+}
+
 // RC_BF16: every row's octets in RC_XR rounds of the workgroup, and the
 // fragments fit LDS beside the kernel's own buffers.
 bool rc_bf16_ok(int qtype, int N, int K, int M, bool pair) {

@@ -323,10 +323,18 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // 5.6 / 5.9 us on the dot kernel) and 9-10 rows (6.76 / 7.00 against 7.27 us
     // in two launches; 12 and 16 rows stay two launches: 7.5 / 8.2 against 7.3
     // us), and for Q5 / Q6 at 8 rows (7.90 / 8.22 against 8.37 / 8.58 us).  W8
-    // keeps 3-4 rows on the dot kernel and 5-8 here.
+    // keeps 3-4 rows on the dot kernel and 5-8 here.  Every round of its
+    // workgroups quantizes the rows again: where the streaming kernel would
+    // take two launches, up to 12 rows times rounds (Q4, K = 7168: 3 rows, N =
+    // 10240 15.6 against 16.5 us, 5 rows, N = 8192 / 10240 13.4 / 18.7 against
+    // 13.5 / 16.5); a pair's two rows up to two rounds (Q5, K = 2048, N = 24576
+    // 23.2 against 21.7 us in two launches).
     const bool q4 = qtype == VIPER_QTYPE_Q4_G64;
     const int bf_max = q4 && !pair ? 10 : 8;
-    const bool rc_bf16 = rc_k && !takes && M <= bf_max && rc_bf16_ok(qtype, N, K, M, pair);
+    int wg_rows;
+    const int rounds = rc_k ? rc_rounds(qtype, pair ? 2L * N : N, K, &wg_rows) : 0;
+    const bool rc_bf16 = rc_k && M <= bf_max && rc_bf16_ok(qtype, N, K, M, pair) && (!takes || (!one && M * rounds <= 12)) &&
+                         !(pair && M == 2 && rounds > 2);
     // Long K splits over workgroups in the two-launch path (down shape
     // K = 10240, 4 rows 9.5 us against 10.3 us without the split), unless one
     // launch serves a K of one phase (Q4, 6 rows, K = 6144, N = 3072 6.8 us
@@ -343,7 +351,12 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // (Q4 rows staged two octets per thread also past that size: down shape
     // K = 10240, 4 rows 8.4 us against 9.0-9.1 us for two launches with the K
     // split)
-    const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M));
+    // (but not where the streaming kernel takes a K of whole quads, the rows
+    // have no exact tiling and there are more than 40 per CU: Q4, 4 rows, K =
+    // 7168, N = 16384 35.6 us against 20.5 in its two launches; 3 rows, K = 9216,
+    // N = 4352 11.4 / 15.3)
+    const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M)) &&
+                         !(takes && rc_k && !m1_rows_exact(qtype, K, M) && N > 40L * device_cus());
     if (rc_bf16 && !split && (M > 4 || !rows_ok || q4)) return R_RC_BF16;
     // (3 or 4 rows here also where the LDS copy does not fit: while every
     // workgroup's share of the rows' quantize stays small; down shape

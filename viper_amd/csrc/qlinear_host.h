@@ -164,6 +164,9 @@ int launch_rc(int qtype, const void* w, const void* s, int senc, int N, int K, c
 // The call's rows (both matrices of a pair) exceed what one workgroup per CU of
 // its row-contiguous kernel holds.
 bool rc_capped(int qtype, long rows_total, int K);
+// Rounds of workgroups, one per CU, the call's rows take there; *rows: rows of a
+// workgroup.
+int rc_rounds(int qtype, long rows_total, int K, int* rows);
 // A split launch's (row, part) pairs exceed two workgroups of 48 rows per CU.
 bool rc_split_capped(int qtype, int N, int K);
 int launch_rc_timeline(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq,
