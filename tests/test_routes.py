@@ -43,3 +43,15 @@ def test_route_k_split(N, K, M, want):
     (Q4, 16384, 7168, 4, 1, STREAM), (Q4, 4352, 9216, 3, 1, ROWS), (Q5, 24576, 2048, 2, 2, RC)])
 def test_route_two_phases(qtype, N, K, M, matrices, want):
     assert route(qtype, BF16, N, K, M, matrices) == want
+
+
+# Two to four rows on the dots or on the matrix cores: exact tilings, two rows at 33..40 per CU, W8's short rows and its
+# few long ones, several phases; int8 rows of a nibble format 3 and 4 on the matrix cores in one round.
+@pytest.mark.parametrize("qtype,rows,N,K,M,want", [
+    (Q4, BF16, 4096, 5120, 2, ROWS), (Q4, BF16, 10240, 5120, 2, ROWS), (Q4, BF16, 2560, 9600, 2, ROWS),
+    (Q4, BF16, 10240, 2112, 2, ROWS), (Q6, BF16, 10240, 2112, 2, ROWS), (W8, BF16, 10240, 1760, 2, ROWS),
+    (Q6, BF16, 8192, 2112, 2, STREAM_BF16), (Q4, BF16, 11005, 4032, 2, STREAM_BF16), (W8, BF16, 16384, 672, 2, ROWS),
+    (W8, BF16, 2560, 3520, 2, ROWS), (W8, BF16, 4256, 4128, 2, ROWS), (W8, BF16, 6144, 3520, 2, STREAM_BF16),
+    (Q4, INT8, 4096, 5120, 4, RC), (Q4, INT8, 28160, 2560, 3, ROWS), (W8, INT8, 2560, 2560, 4, ROWS)])
+def test_route_dots(qtype, rows, N, K, M, want):
+    assert route(qtype, rows, N, K, M) == want

@@ -270,24 +270,27 @@ static int validate_second(const Second& b, int qtype, int senc, int group, int 
 }
 
 // Two to four rows of one matrix: on the M = 1 kernel's dot path, or on the
-// matrix cores?  The dot path's exact tilings (K = 2560: 2 rows 3.6 us against
-// 4.2 at N = 2560), and K beyond one phase of the streaming kernel, where its
-// serial phases or a second launch cost more (one: K has one phase; Q4, 2
-// rows, N = 2560, dot / matrix cores: K = 9600 8.9 / 11.7; K = 6144 7.3 / 5.0,
-// K = 4096 6.9 / 4.1, K = 1984 5.5 / 4.0, K = 512 4.3 / 2.7; 4 rows K = 4096,
-// N = 10240 11.2 / 9.0).  Two rows of the formats that decode cheapest stay on
-// the dots also where short rows are many (K = 2048, N = 20480: Q4 8.4 / 9.7,
-// W8 12.9 / 13.4; N = 8192 5.6 / 4.3, 6.8 / 6.7; K = 3520, where 40 rows per CU are
-// two and a half tiles, N = 10240: Q4 8.2 / 8.7) and where W8's kernel has its
-// most registers and one tile a workgroup (K = 3520, N = 2560 6.3 / 6.5;
-// N = 6144 11.0 / 9.7).
-static bool dot_rows(int qtype, int N, int K, int M, bool one) {
+// matrix cores?  The dot path's exact multi-row tilings (K = 2560, 5120, 10240:
+// Q4, 2 rows, K = 5120, N = 4096 / 10240 4.4 / 7.4 us against 4.7 / 10.2), and K
+// beyond one phase of the streaming kernel, where its serial phases or a
+// second launch cost more (one: K has one phase; Q4, 2 rows, N = 2560, dot /
+// matrix cores: K = 9600 8.9 / 11.7; K = 6144 7.3 / 5.0, K = 4096 6.9 / 4.1,
+// K = 3072 6.4 / 3.7, K = 512 4.3 / 2.7; 4 rows K = 4096, N = 10240 11.2 / 9.0).
+// Two rows also where the streaming kernel (takes) would fill its last tile
+// least while one round of 40-row workgroups holds them here, 33..40 rows per
+// CU (N = 10240: Q4 K = 2112 5.6 / 6.5, K = 4608 8.1 / 9.7; Q6 K = 2112 6.9 / 7.7;
+// W8 K = 1760 5.4 / 6.2; N = 8192 the other way; Q4, K = 4096, N = 11005, two
+// rounds, 12.3 / 8.2), short rows of W8, which decodes cheapest, from there on
+// (N = 16384, K = 704 4.8 / 5.8, K = 1056 5.9 / 6.7), and few long ones of it,
+// whose tiles take the most steps (K = 3520, N = 2560 6.3 / 6.5; K = 4096, N =
+// 4256 6.7 / 8.9, N = 6144 equal).
+static bool dot_rows(int qtype, int N, int K, int M, bool one, bool takes) {
     if (!m1_rows_ok(qtype, K, M)) return false;
     if (m1_rows_exact(qtype, K, M) || !one) return true;
+    if (M > 2 || !takes) return false;
     const bool w8 = qtype == VIPER_QTYPE_W8_G32;
     const long per_cu = (N + (long)device_cus() - 1) / device_cus();
-    if (M > 2 || !(w8 || qtype == VIPER_QTYPE_Q4_G64)) return false;
-    return (per_cu > 32 && (K <= 2048 || (per_cu <= 48 && !rc_ok(qtype, K)))) || (w8 && K > 96 * 32 && !rc_ok(qtype, K) && per_cu <= 16);
+    return (per_cu > 32 && (per_cu <= 40 || (w8 && K <= 1152))) || (w8 && K > 96 * 32 && per_cu <= 20);
 }
 
 // The kernel a call runs, from its sizes alone (the routes of include/viper_qlinear.h).
@@ -316,7 +319,7 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // N = 2560 6.1 / 7.0, N = 10240 9.8 / 10.6; K = 4096, N = 10240 9.9 / 10.6).
     const bool one = sg_bf16_ok(qtype, N, K, M, pair);
     const bool takes = sg_takes(qtype, N, K, pair);
-    const bool dot = !pair && dot_rows(qtype, N, K, M, one);
+    const bool dot = !pair && dot_rows(qtype, N, K, M, one, takes);
     if (M == 2 && dot) return R_ROWS;
     // With the rows staged two octets per thread (64-groups), the row-contiguous
     // kernel's one-launch path also wins for Q4 at 3-4 rows (5.45 / 5.74 against
@@ -356,7 +359,7 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // 7168, N = 16384 35.6 us against 20.5 in its two launches; 3 rows, K = 9216,
     // N = 4352 11.4 / 15.3)
     const bool rows_ok = dot && ((long)M * K <= 32768 || m1_rows_pair(qtype, K, M)) &&
-                         !(takes && rc_k && !m1_rows_exact(qtype, K, M) && N > 40L * device_cus());
+                         !(takes && (one || (rc_k && !m1_rows_exact(qtype, K, M) && N > 40L * device_cus())));
     if (rc_bf16 && !split && (M > 4 || !rows_ok || q4)) return R_RC_BF16;
     // (3 or 4 rows here also where the LDS copy does not fit: while every
     // workgroup's share of the rows' quantize stays small; down shape
@@ -371,11 +374,16 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
 // int8 rows in the layout of viper_hip_quantize_act.
 static Route prequant_route(int qtype, int N, int K, int M, bool pair) {
     if (fused_ok(qtype, M, K)) return R_M1;
-    const bool one = sg_phases(qtype, K, RC_NAT) == 1;
-    // (a K of whole group quads has no workgroup quantize here: on the matrix
-    // cores it is faster at many rows too, Q4 K = 2048, 2 rows, N = 10240 6.3 / 5.1)
-    if (!pair && dot_rows(qtype, N, K, M, one) && (m1_rows_exact(qtype, K, M) || !one || !rc_ok(qtype, K))) return R_ROWS;
-    return M < 2 || sg_takes(qtype, N, K, pair) ? R_SG : R_RC;
+    const bool one = sg_phases(qtype, K, RC_NAT) == 1, takes = sg_takes(qtype, N, K, pair);
+    const bool rc_k = M >= 2 && rc_ok(qtype, K);
+    // (3 and 4 rows of a nibble format and K of one phase: the matrix cores, also
+    // against an exact tiling, Q4, 4 rows, K = 5120, N = 512 / 4096 4.6 / 5.4 us
+    // against 5.2 / 5.9; not in several rounds, 3 rows, K = 2560, N = 28160 13.8
+    // against 11.4)
+    int wg_rows;
+    const bool rows34 = M > 2 && one && rc_k && qtype != VIPER_QTYPE_W8_G32 && (takes || rc_rounds(qtype, N, K, &wg_rows) == 1);
+    if (!pair && !rows34 && dot_rows(qtype, N, K, M, one, takes)) return R_ROWS;
+    return M < 2 || takes ? R_SG : R_RC;
 }
 
 // int8 fragments; ws: with a workspace the K split may use.
