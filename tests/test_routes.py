@@ -55,3 +55,13 @@ def test_route_two_phases(qtype, N, K, M, matrices, want):
     (Q4, INT8, 4096, 5120, 4, RC), (Q4, INT8, 28160, 2560, 3, ROWS), (W8, INT8, 2560, 2560, 4, ROWS)])
 def test_route_dots(qtype, rows, N, K, M, want):
     assert route(qtype, rows, N, K, M) == want
+
+
+# Past one round of the row-contiguous kernel: the streaming kernel, but for equal padding with part of a step of four
+# groups idle, and two bf16 rows also before it where it pads fewer rows.
+@pytest.mark.parametrize("qtype,rows,N,K,M,matrices,want", [
+    (Q4, BF16, 14336, 3328, 4, 1, RC_BF16), (Q4, BF16, 14336, 4096, 4, 1, STREAM_BF16), (Q4, INT8, 16384, 4608, 16, 1, RC),
+    (Q4, FRAG, 14336, 3328, 16, 1, STREAM), (Q4, INT8, 13312, 3584, 7, 2, STREAM), (Q6, BF16, 10000, 3328, 4, 1, STREAM_BF16),
+    (Q5, BF16, 14000, 2048, 2, 1, STREAM_BF16), (Q4, BF16, 14000, 2048, 3, 1, RC_BF16)])
+def test_route_padding(qtype, rows, N, K, M, matrices, want):
+    assert route(qtype, rows, N, K, M, matrices) == want

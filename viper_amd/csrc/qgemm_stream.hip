@@ -51,12 +51,11 @@ bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair) {
     return sg_launch(qtype, sg_rows(N, pair), K, M, RC_BF16, false, 0, l) && l.np == 1;
 }
 
-// Which calls the streaming kernel takes: K that the row-contiguous kernel
-// cannot (not a multiple of four groups), and K whose row-contiguous kernel
-// holds fewer rows per CU than the call has (its two-quad and segment-loop
-// kernels, see rc_capped), where it ran the chip in several rounds of
-// workgroups (fragments, M = 16, us, row-contiguous / streaming: Q4 N = 10240
-// K = 4096 12.2 / 9.0, K = 5120 13.7 / 10.9, K = 6144 19.3 / 11.7; Q5
+// Which calls of whole group quads the streaming kernel takes from the
+// row-contiguous kernel: those whose rows exceed one round of its workgroups
+// (its two-quad and segment-loop kernels, see rc_capped), where that ran the
+// chip in several rounds (fragments, M = 16, us, row-contiguous / streaming: Q4
+// N = 10240 K = 4096 12.2 / 9.0, K = 5120 13.7 / 10.9, K = 6144 19.3 / 11.7; Q5
 // N = 10240 K = 4096 13.7 / 10.3; Q6 13.2 / 11.4; W8 N = 10240 K = 3072 16.3 /
 // 11.0; and where it holds them: Q4 N = 5120 K = 4096 6.4 / 6.8, K = 5120
 // 7.0 / 8.3, N = 10240 K = 3072 6.4 / 7.7).
@@ -64,9 +63,29 @@ bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair) {
 // 40.8 / 30.6): serial phases cost more than rounds of workgroups (Q5, four
 // phases, K = 12800, N = 6400, M = 6 26.1 / 29.2; K = 12544, N = 7815, M = 3
 // 26.6 / 29.4).
-bool sg_takes(int qtype, int N, int K, bool pair) {
+// Where both kernels' rounds cover the same padded rows (16-row tiles here, its
+// workgroups' rows there) and the waves' groups leave part of a step of four
+// idle, up to 4 bf16 rows of Q4 and more than 8 int8 rows of all but Q6 stay
+// there (Q4, N = 13312..16384, row-contiguous / streaming: 4 bf16 rows of K =
+// 3328 9.7 / 10.5, 16 int8 rows of K = 4608 14.4 / 16.3; of K = 4096, whole steps,
+// 13.9 / 11.9; fragments of K = 3328 10.4 / 10.0, 7 int8 rows of a pair of K =
+// 3584 20.8 / 18.6; Q6, N = 10000, 4 bf16 rows of K = 3328 12.1 / 10.7).
+// Two bf16 rows also leave the other kernels of that family for one that pads
+// fewer rows (Q5, K = 2048, N = 14000 11.3 / 8.3; Q4 8.1 / 7.5).
+bool sg_takes(int qtype, int N, int K, int M, bool pair, int am) {
     if (!rc_ok(qtype, K)) return true;
-    return sg_phases(qtype, K, RC_FRAG) <= (qtype == VIPER_QTYPE_Q4_G64 ? 2 : 1) && rc_capped(qtype, sg_rows(N, pair), K);
+    const long total = sg_rows(N, pair);
+    const int phases = sg_phases(qtype, K, RC_FRAG);
+    if (phases > (qtype == VIPER_QTYPE_Q4_G64 ? 2 : 1)) return false;
+    int rows;
+    const int rounds = rc_rounds(qtype, total, K, &rows);
+    const long per_cu = (total + device_cus() - 1) / device_cus();
+    if (!rc_capped(qtype, total, K))
+        return am == RC_BF16 && M == 2 && !pair && rounds > 1 && (per_cu + 15) / 16 * 16 < (long)rounds * rows;
+    const int gw = (K / group_of(qtype) + SG_W - 1) / SG_W;
+    const bool even = rows > 16 && (per_cu + 15) / 16 * 16 == (long)rounds * rows && gw % 4 != 0;
+    return !(even && !pair && ((am == RC_NAT && M > 8 && qtype != VIPER_QTYPE_Q6_G64) ||
+                               (am == RC_BF16 && M <= 4 && qtype == VIPER_QTYPE_Q4_G64)));
 }
 
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,

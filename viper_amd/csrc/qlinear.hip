@@ -318,7 +318,7 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // quantizes up to 8 rows itself (Q4, M = 8, us, one launch / two: K = 3520,
     // N = 2560 6.1 / 7.0, N = 10240 9.8 / 10.6; K = 4096, N = 10240 9.9 / 10.6).
     const bool one = sg_bf16_ok(qtype, N, K, M, pair);
-    const bool takes = sg_takes(qtype, N, K, pair);
+    const bool takes = sg_takes(qtype, N, K, M, pair, one ? RC_BF16 : RC_FRAG);
     const bool dot = !pair && dot_rows(qtype, N, K, M, one, takes);
     if (M == 2 && dot) return R_ROWS;
     // With the rows staged two octets per thread (64-groups), the row-contiguous
@@ -374,7 +374,7 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
 // int8 rows in the layout of viper_hip_quantize_act.
 static Route prequant_route(int qtype, int N, int K, int M, bool pair) {
     if (fused_ok(qtype, M, K)) return R_M1;
-    const bool one = sg_phases(qtype, K, RC_NAT) == 1, takes = sg_takes(qtype, N, K, pair);
+    const bool one = sg_phases(qtype, K, RC_NAT) == 1, takes = sg_takes(qtype, N, K, M, pair, RC_NAT);
     const bool rc_k = M >= 2 && rc_ok(qtype, K);
     // (3 and 4 rows of a nibble format and K of one phase: the matrix cores, also
     // against an exact tiling, Q4, 4 rows, K = 5120, N = 512 / 4096 4.6 / 5.4 us
@@ -388,7 +388,7 @@ static Route prequant_route(int qtype, int N, int K, int M, bool pair) {
 
 // int8 fragments; ws: with a workspace the K split may use.
 static Route frag_route(int qtype, int N, int K, int M, bool pair, bool ws) {
-    const bool takes = sg_takes(qtype, N, K, pair);
+    const bool takes = sg_takes(qtype, N, K, M, pair, RC_FRAG);
     if (ws && !pair && frag_workspace_need(qtype, N, K, M) > 0 && !(takes && rc_split_capped(qtype, N, K))) return R_SPLIT;
     return takes ? R_SG : R_RC;
 }

@@ -175,7 +175,7 @@ int launch_rc_timeline(int qtype, const void* w, const void* s, int senc, int N,
 
 // M = 1..16, any K (qgemm_stream.hip): persistent workgroups, the activation
 // operands in registers.  am as for launch_rc; part only with RC_FRAG.
-bool sg_takes(int qtype, int N, int K, bool pair);
+bool sg_takes(int qtype, int N, int K, int M, bool pair, int am);
 int sg_phases(int qtype, int K, int am);  // over K: what one workgroup's waves hold in registers
 bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair);
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
