@@ -334,6 +334,7 @@ int viper_hip_check_quantizer(int exp_lo, int exp_hi, int32_t* counts, void* str
 #define VIPER_ROUTE_RC_SPLIT 4    /* the row-contiguous kernel's K split */
 #define VIPER_ROUTE_RC 5          /* the row-contiguous kernel on int8 rows */
 #define VIPER_ROUTE_STREAM 6      /* the streaming kernel on int8 rows */
+#define VIPER_ROUTE_PAIRS 7       /* the matrix-core kernel that gathers group pairs, on int8 rows */
 int viper_hip_qlinear_route(int qtype, int input, int N, int K, int M, int matrices);
 
 /* Measurement entry point, no counterpart in the reference: the M = 1 GEMV

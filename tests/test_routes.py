@@ -6,7 +6,7 @@ import viper_amd as va
 
 Q4, Q5, Q6, W8 = 4, 5, 6, 8
 BF16, INT8, FRAG = 0, 1, 2
-M1, ROWS, RC_BF16, STREAM_BF16, RC_SPLIT, RC, STREAM = range(7)
+M1, ROWS, RC_BF16, STREAM_BF16, RC_SPLIT, RC, STREAM, PAIRS = range(8)
 
 
 def route(qtype, rows, N, K, M, matrices=1):
@@ -65,3 +65,15 @@ def test_route_dots(qtype, rows, N, K, M, want):
     (Q5, BF16, 14000, 2048, 2, 1, STREAM_BF16), (Q4, BF16, 14000, 2048, 3, 1, RC_BF16)])
 def test_route_padding(qtype, rows, N, K, M, matrices, want):
     assert route(qtype, rows, N, K, M, matrices) == want
+
+
+# K of an even number of groups, not a multiple of four: gathered pairs for short rows, few rows per CU and many rows of
+# the formats that decode cheapest; the streaming kernel else.
+@pytest.mark.parametrize("qtype,rows,N,K,M,want", [
+    (Q4, BF16, 2048, 384, 16, PAIRS), (Q4, INT8, 2048, 384, 16, PAIRS), (Q4, INT8, 256, 384, 16, STREAM),
+    (Q4, BF16, 2048, 4224, 16, PAIRS), (Q6, BF16, 6144, 4224, 8, PAIRS), (Q4, BF16, 24000, 3712, 16, PAIRS),
+    (W8, BF16, 24000, 2112, 16, PAIRS), (W8, BF16, 10240, 2112, 16, STREAM), (Q4, BF16, 2048, 8320, 16, PAIRS),
+    (Q5, BF16, 2048, 6784, 16, STREAM), (Q4, INT8, 2048, 8320, 16, PAIRS), (Q4, INT8, 2048, 8320, 8, STREAM),
+    (W8, BF16, 256, 13248, 12, STREAM), (Q4, BF16, 24576, 384, 8, PAIRS), (Q4, BF16, 2560, 3456, 8, STREAM_BF16)])
+def test_route_pairs(qtype, rows, N, K, M, want):
+    assert route(qtype, rows, N, K, M) == want

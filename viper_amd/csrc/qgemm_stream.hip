@@ -88,6 +88,45 @@ bool sg_takes(int qtype, int N, int K, int M, bool pair, int am) {
                                (am == RC_BF16 && M <= 4 && qtype == VIPER_QTYPE_Q4_G64)));
 }
 
+// K of an even number of groups, not a multiple of four: this kernel, or the
+// one that gathers group pairs (qgemm_mfma.hip)?  That one has the shorter
+// chain after a workgroup's weights arrive (no LDS transpose, four waves up to
+// 40 groups, one load segment up to 80) and as many workgroups as there are
+// row blocks; this one streams.  So it takes, us, pairs / streaming:
+//  * short rows: up to 24 groups (Q4, M = 16, K = 384, N = 2048 / 24576, two
+//    launches 3.9 / 4.5 and 7.2 / 10.3; int8 rows 2.1 / 2.3, 5.7 / 7.5, but N =
+//    256 the other way by 6 %), up to 40 after a quantize launch, for W8, or for
+//    at most 16 rows per CU;
+//  * few rows per CU (16) where one load segment of it holds what this kernel
+//    needs more steps for (Q4, M = 16, N = 2048, K = 4224 6.0 / 6.8; Q6, M = 8
+//    8.3 / 9.5, and there, in two phases, up to 40: N = 6144 12.0 / 13.3);
+//  * 9 and more rows of Q4 / W8 over many short rows, more tiles than its waves
+//    can hide (M = 16, N = 24000, K = 3712 18.5 / 20.2 with a residual, W8, K =
+//    2112 18.1 / 23.0; N = 10240 the other way);
+//  * few rows per CU and a K of several phases (Q4, M = 16, N = 2048, K = 8320
+//    11.0 / 13.3), where those are not nearly full (Q5, K = 6784 10.0 / 9.6).  Of
+//    int8 rows, which that kernel gathers, only 9 and more of 128 groups (Q4,
+//    M = 16, K = 8320 1.06 times, M = 8 0.98; K = 7552 8.4 against 9.9 here).
+// Never for more groups than its staged scales hold (W8, M = 12, K = 13248, N =
+// 256 25.7 / 20.5).  A call of one launch here (up to 8 bf16 rows of one phase) is compared with
+// its two: there only many short rows (Q4, K = 384, N = 24576, M = 8 9.0 / 10.4;
+// N = 16384 equal) and many values a workgroup quantizes (Q4, M = 8, K = 4224,
+// N = 2048 6.6 / 7.3).
+bool sg_over_mf(int qtype, int N, int K, int M, bool pair, int am) {
+    if (M < 2 || !mf_ok(qtype, K)) return true;
+    const int NG = K / group_of(qtype), F = qtype == VIPER_QTYPE_W8_G32 ? 8 : qtype;
+    const long per_cu = (sg_rows(N, pair) + device_cus() - 1) / device_cus();
+    const bool wide = F == 5 || F == 6, nat = am == RC_NAT;
+    if (nat ? NG > 384 || per_cu <= 1 : !mf_frag_ok(qtype, N, K)) return true;
+    if (am == RC_BF16) return !((NG <= (wide ? 12 : F == 8 ? 24 : 40) && per_cu > 80) || ((long)M * K >= 32768 && per_cu <= 16));
+    if (NG <= 40 && (per_cu <= 16 || NG <= (wide && nat ? 8 : 24) || !nat || F == 8)) return false;
+    if (NG > 64 && NG <= 80 && per_cu <= (wide && !nat ? 40 : 16)) return false;
+    if (!nat && M > 8 && !wide && NG <= 80 && per_cu > (F == 8 ? 48 : 80)) return false;
+    const int phases = sg_phases(qtype, K, am), cap = phases * SG_W * 2 * sg_ni_max(F, am, false);
+    if (phases == 1 || per_cu > 16) return true;
+    return nat ? M <= 8 || wide || NG < 128 : wide && NG * 20 >= cap * (phases == 2 ? 15 : 16);
+}
+
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
               int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1, hipStream_t st) {
     const bool pair = w1 != nullptr;

@@ -302,6 +302,7 @@ enum Route {
     R_SPLIT = VIPER_ROUTE_RC_SPLIT,
     R_RC = VIPER_ROUTE_RC,
     R_SG = VIPER_ROUTE_STREAM,
+    R_MF = VIPER_ROUTE_PAIRS,
 };
 
 // bf16 rows.  Few rows: every workgroup quantizes the rows itself, one launch
@@ -367,8 +368,9 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // split)
     if (rows_ok) return R_ROWS;
     if (split) return R_SPLIT;
-    if (takes && one && !part) return R_SG_BF16;
-    return takes ? R_SG : R_RC;
+    if (takes && one && !part && sg_over_mf(qtype, N, K, M, pair, RC_BF16)) return R_SG_BF16;
+    if (rc_k) return takes ? R_SG : R_RC;
+    return sg_over_mf(qtype, N, K, M, pair, RC_FRAG) ? R_SG : R_MF;
 }
 
 // int8 rows in the layout of viper_hip_quantize_act.
@@ -383,7 +385,8 @@ static Route prequant_route(int qtype, int N, int K, int M, bool pair) {
     int wg_rows;
     const bool rows34 = M > 2 && one && rc_k && qtype != VIPER_QTYPE_W8_G32 && (takes || rc_rounds(qtype, N, K, &wg_rows) == 1);
     if (!pair && !rows34 && dot_rows(qtype, N, K, M, one, takes)) return R_ROWS;
-    return M < 2 || takes ? R_SG : R_RC;
+    if (rc_k) return takes ? R_SG : R_RC;
+    return sg_over_mf(qtype, N, K, M, pair, RC_NAT) ? R_SG : R_MF;
 }
 
 // int8 fragments; ws: with a workspace the K split may use.
@@ -435,10 +438,13 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     // the workspace's start, then the records of part sums)
     uint64_t* sp = route == R_SPLIT ? (uint64_t*)((uint8_t*)wsp + lay.sp) : nullptr;
     unsigned* sc = route == R_SPLIT ? (unsigned*)wsp : nullptr;
-    rc = launch_quantize(group, x, M, K, xq, xs, true, st);
+    const bool nat = route == R_MF && !mf_frag_ok(qtype, N, K);
+    rc = launch_quantize(group, x, M, K, xq, xs, !nat, st);
     if (rc != VIPER_OK) return rc;
     if (route == R_SG)
         return launch_sg(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st);
+    if (route == R_MF)
+        return launch_mf(qtype, w, s, senc, N, K, xq, xs, nat, M, y, res, part, b.w, b.s, b.y, st);
     return launch_rc(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st, sp, sc);
 }
 
@@ -461,6 +467,8 @@ static int prequant_common(int qtype, const void* w, const void* s, int senc, in
     if (rows_refused(qtype, M, K)) return VIPER_INVALID_ARGUMENT;
     if (route == R_SG)
         return launch_sg(qtype, w, s, senc, N, K, xq, xs, RC_NAT, M, y, res, nullptr, b.w, b.s, b.y, st);
+    if (route == R_MF)
+        return launch_mf(qtype, w, s, senc, N, K, xq, xs, true, M, y, res, nullptr, b.w, b.s, b.y, st);
     return launch_rc(qtype, w, s, senc, N, K, xq, xs, RC_NAT, M, y, res, nullptr, b.w, b.s, b.y, st);
 }
 

@@ -173,9 +173,18 @@ int launch_rc_timeline(int qtype, const void* w, const void* s, int senc, int N,
                        const void* xs, int M, void* y, uint64_t* stamps, size_t stamp_bytes, int* workgroups,
                        int* waves, unsigned* sc, hipStream_t st);
 
+// M = 2..16, K a multiple of two groups but not of four (qgemm_mfma.hip): group
+// pairs gathered straight into the matrix-core layout.  xnat: activations in
+// the natural layout, else in fragment order (mf_frag_ok must hold).
+bool mf_ok(int qtype, int K);
+bool mf_frag_ok(int qtype, int N, int K);
+int launch_mf(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, bool xnat,
+              int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1, hipStream_t st);
+
 // M = 1..16, any K (qgemm_stream.hip): persistent workgroups, the activation
 // operands in registers.  am as for launch_rc; part only with RC_FRAG.
 bool sg_takes(int qtype, int N, int K, int M, bool pair, int am);
+bool sg_over_mf(int qtype, int N, int K, int M, bool pair, int am);
 int sg_phases(int qtype, int K, int am);  // over K: what one workgroup's waves hold in registers
 bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair);
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
