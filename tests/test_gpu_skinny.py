@@ -14,7 +14,7 @@ import oracle as O
 import viper_amd as va
 from test_gpu_folded import dev, u16, weights
 from test_gpu_frag import to_frag
-from test_gpu_parity import run_case, torch_dev  # noqa: F401
+from test_gpu_parity import REL_TOL, run_case, torch_dev  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 FORMATS = [O.Q4_G64, O.Q5_G64, O.Q6_G64, O.W8_G32]
@@ -100,3 +100,25 @@ def test_skinny_nonfinite_stays(torch_dev, M):  # noqa: F811
     keep[:, 33] = False
     keep[1, :] = False
     np.testing.assert_array_equal(a[keep], b[keep])
+
+
+# The residual's values are requested by the wave that sums a tile: one to many tiles per workgroup, a ragged last one,
+# rows short of 16, one and several phases, in place and apart, against the oracle.
+@pytest.mark.parametrize("qtype,N,ng,M", [(O.Q4_G64, 15, 5, 3), (O.Q4_G64, 23260, 5, 10), (O.Q4_G64, 11000, 96, 16),
+                                          (O.Q5_G64, 12289, 3, 9), (O.Q6_G64, 517, 101, 5), (O.W8_G32, 9001, 61, 7),
+                                          (O.W8_G32, 300, 121, 12)])
+def test_skinny_residual(torch_dev, qtype, N, ng, M):  # noqa: F811
+    torch = torch_dev
+    G = O.group_size(qtype)
+    K = ng * G
+    w, packed, scales = weights(torch, qtype, N, K, 0x5C5000 + N, O.SCALE_BF16)[:3]
+    x, res = O.gen_act(M, K, 0x5C5010, outlier_frac=0.02), O.gen_act(M, N, 0x5C5011)
+    rd, y = dev(torch, res), torch.zeros((M, N), dtype=torch.int16, device="cuda")
+    wk = torch.zeros(max(16, va.workspace_bytes(qtype, N, K, M)), dtype=torch.uint8, device="cuda")
+    z = rd.clone()
+    assert va.linear(w, dev(torch, x), y, residual=rd, workspace=wk).ok()
+    assert va.linear(w, dev(torch, x), z, residual=z, workspace=wk).ok()
+    torch.cuda.synchronize()
+    y_ref, _, absterm = O.qlinear(qtype, packed, scales, O.SCALE_BF16, N, K, x, residual=res)
+    O.assert_bf16_close(u16(y), y_ref, absterm, rel=REL_TOL)
+    np.testing.assert_array_equal(u16(y), u16(z))
