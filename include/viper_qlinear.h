@@ -381,7 +381,10 @@ int viper_hip_stream_read(const void* buf, size_t bytes, int threads, int loads,
  * outputs stored (y by the K split's last part of a block); readings a
  * workgroup does not reach repeat its last one.  *workgroups and
  * *waves_per_workgroup (may be NULL) receive the grid; stamp_bytes must
- * cover it.  y equals the production call's bit for bit. */
+ * cover it.  Calls that the streaming kernel serves (VIPER_ROUTE_STREAM) are
+ * traced there, per tile of 16 rows: weight loads issued, scales in LDS and
+ * first group of the first tile, last group, barrier and sums of the last.
+ * y equals the production call's bit for bit. */
 int viper_hip_qlinear_frag_timeline(int qtype, const void* w_packed, const void* w_scales, int scale_enc, int group,
                                     int N, int K, const void* xfrag, const void* xsfrag, int M, void* y_bf16,
                                     uint64_t* stamps, size_t stamp_bytes, int* workgroups, int* waves_per_workgroup,

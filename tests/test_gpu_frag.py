@@ -378,3 +378,38 @@ def test_frag_timeline_matches_gemm(torch_dev, M, K, N):
                                                  st) == 2
         assert L.viper_hip_qlinear_frag_timeline(4, *args, stamps.data_ptr(), stamps.numel() * 8, None, None, wsp,
                                                  nws - 16, st) == 2
+
+
+# the timeline where the production call runs the streaming kernel (rows past the row-contiguous kernel's one round): the
+# same bits, non-decreasing readings of every wave, the refusals as before
+@pytest.mark.parametrize("qtype,M,K,N", [(O.Q4_G64, 16, 4096, 10240), (O.Q4_G64, 7, 5120, 10007), (O.Q4_G64, 3, 3328, 16400),
+                                         (O.W8_G32, 16, 2560, 20000), (O.W8_G32, 8, 2304, 20011)])
+def test_frag_timeline_matches_streaming(torch_dev, qtype, M, K, N):
+    import ctypes as C
+    torch = torch_dev
+    L = va.lib()
+    G = O.group_size(qtype)
+    assert L.viper_hip_qlinear_route(qtype, 2, N, K, M, 1) == 6
+    packed, scales = O.gen_weights(qtype, N, K, 760 + M, O.SCALE_BF16)
+    w = va.QuantizedWeight(va.QType(qtype), dev(torch, packed), dev(torch, scales), N, K, G, va.ScaleEnc.BF16)
+    xf, sf = _frag_buffers(torch, K, G)
+    assert va.rmsnorm_quantize_frag(dev(torch, O.gen_act(M, K, 761)), dev(torch, bf16(np.ones(K))), 1e-6, G, xf, sf).ok()
+    y0 = torch.zeros((M, N), dtype=torch.int16, device="cuda")
+    y1 = torch.full((M, N), 7, dtype=torch.int16, device="cuda")
+    assert va.linear_prequantized_frag(w, xf, sf, y0).ok()
+    stamps = torch.zeros(10 << 14, dtype=torch.int64, device="cuda")
+    grid, waves = C.c_int(0), C.c_int(0)
+    st = torch.cuda.current_stream().cuda_stream
+    args = (qtype, w.data.data_ptr(), w.scales.data_ptr(), 1, G, N, K, xf.data_ptr(), sf.data_ptr(), M, y1.data_ptr())
+    assert L.viper_hip_qlinear_frag_timeline(*args, stamps.data_ptr(), stamps.numel() * 8, C.byref(grid), C.byref(waves),
+                                             None, 0, st) == 0
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(u16(y1), u16(y0))
+    nw = grid.value * waves.value
+    t = stamps.view(-1, 10)[:nw].cpu().numpy()
+    assert nw > 0 and (np.diff(t, axis=1) >= 0).all() and (t[:, 0] > 0).all() and (t[:, 9] == t[:, 7]).all()
+    assert (stamps.view(-1)[nw * 10:] == 0).all()
+    assert L.viper_hip_qlinear_frag_timeline(*args, stamps.data_ptr(), nw * 80 - 8, None, None, None, 0, st) == 2
+    wk = torch.zeros(64, dtype=torch.uint8, device="cuda")  # a workspace where there is no split stays refused
+    assert L.viper_hip_qlinear_frag_timeline(*args, stamps.data_ptr(), stamps.numel() * 8, None, None, wk.data_ptr(), 64,
+                                             st) == 2

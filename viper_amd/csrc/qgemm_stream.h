@@ -103,14 +103,21 @@ __host__ __device__ constexpr size_t sg_act_lds(int g, int rows, int ng) { retur
 // workgroups per XCD in bits 12..31.  AM, as in qgemm_rc.h: RC_FRAG, RC_NAT or
 // RC_BF16 (xq = x; one phase).  PK: groups per accumulator, 2 for M <= 8, else
 // 1.  SE: scale encoding, 2 = from ms.  PART: also store every int32 group dot
-// (test and debug entry point).
-template <int F, int NI, int PK, int AM, int SE, bool PART>
+// (test and debug entry point).  TLM (measurement): `part` receives per-wave
+// timestamps instead, as in qgemm_rc.h.
+template <int F, int NI, int PK, int AM, int SE, bool PART, bool TLM = false>
 __global__ void __launch_bounds__(64 * SG_W)
 qgemm_stream_kernel(const int8_t* xq, const float* xs, const uint8_t* w, const uint16_t* ws, uint16_t* y, unsigned kk,
                     int N, unsigned rg, unsigned ms, const uint16_t* res, int32_t* __restrict__ part, const uint8_t* w1,
                     const uint16_t* ws1, uint16_t* y1) {
     using SH = SgShape<F, NI>;
     using Tile = typename SH::Tile;
+    static_assert(!TLM || (!PART && AM == RC_FRAG), "timeline: fragment input");
+    uint64_t tstamp[RC_TL_STAMPS];
+    auto stamp = [&](int i) {
+        if constexpr (TLM) tstamp[i] = __builtin_amdgcn_s_memrealtime();
+    };
+    stamp(0);
     constexpr int G = F == 8 ? 32 : 64, QB = F == 8 ? 8 : 16, HB = SH::HB, W = SG_W, NTT = 64 * SG_W, GWX = SH::GWX, NH = SH::NH, NS = SH::NS;
     constexpr int R2 = 16 / PK;               // columns per group: the rows of x, rounded up
     constexpr int NPK = (GWX + PK - 1) / PK;  // accumulator groups per wave and phase
@@ -302,8 +309,10 @@ qgemm_stream_kernel(const int8_t* xq, const float* xs, const uint8_t* w, const u
     } else {
         act_load();
         issue_fence();
+        stamp(1);
         load(T0, 0);
         issue_fence();
+        stamp(2);
     }
     // scales past the wave's groups stay zero (their products must be finite)
     for (int i = lane; i < SH::SCB / 4; i += 64) ((uint32_t*)sb)[i] = 0u;
@@ -350,6 +359,7 @@ qgemm_stream_kernel(const int8_t* xq, const float* xs, const uint8_t* w, const u
                 }
         }
         wave_sync();
+        if (TLM && t == 0 && p == 0) stamp(3);
         const bool sums = (t & (W - 1)) == wave, add = res != nullptr && p + 1 == NP;
         const size_t o0 = (size_t)n16 * N + row0 + 4 * kb;
         uint16_t rv[4] = {0, 0, 0, 0};
@@ -420,7 +430,9 @@ qgemm_stream_kernel(const int8_t* xq, const float* xs, const uint8_t* w, const u
                     }
                 }
             }
+            if (TLM && h0 == 0 && t == 0 && p == 0) stamp(4);
         }
+        stamp(5);
         // the pack's groups, then the waves in order (two buffers in turn: one
         // barrier per tile), by one wave, in turn
         float* rd = red + rb * (W * 256);
@@ -431,6 +443,8 @@ qgemm_stream_kernel(const int8_t* xq, const float* xs, const uint8_t* w, const u
         }
         *(float4*)(rd + (wave * 64 + lane) * 4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
         lds_barrier();
+        stamp(6);
+        stamp(7);
         if (!sums) return;
         float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -457,6 +471,7 @@ qgemm_stream_kernel(const int8_t* xq, const float* xs, const uint8_t* w, const u
                 }
             }
         }
+        stamp(7);
     };
     for (int p = 0;;) {
         // (separate code for the last tile, so that no wait counts loads that
@@ -490,6 +505,15 @@ qgemm_stream_kernel(const int8_t* xq, const float* xs, const uint8_t* w, const u
         wave_sync();
         for (int i = lane; i < SH::SCB / 4; i += 64) ((uint32_t*)sb)[i] = 0u;
         act_ready();
+    }
+    if constexpr (TLM) {
+        // (no second matrix: bid counts the workgroups that have rows; the
+        // points of the K split repeat the last one)
+        if (lane == 0) {
+            uint64_t* o = (uint64_t*)part + ((size_t)bid * W + wave) * RC_TL_STAMPS;
+#pragma unroll
+            for (int i = 0; i < RC_TL_STAMPS; ++i) o[i] = tstamp[i < 7 ? i : 7];
+        }
     }
 }
 
@@ -534,6 +558,22 @@ sg_fn sg_pick(int gw, int am, bool pack, bool part, int senc, size_t* lds) {
 #undef VQ_SG
     return nullptr;
 }
+
+// Timeline kernels (fragments; the groups per wave of K past one quad of the
+// row-contiguous kernel, whose measurement entry point launches them).
+template <int F>
+sg_fn sg_pick_tl(int gw, bool pack) {
+#define VQ_SG_TL(NI_)                                           \
+    if constexpr (NI_ <= sg_ni_max(F, RC_FRAG, false))          \
+        if (gw <= 2 * NI_)                                      \
+            return pack ? qgemm_stream_kernel<F, NI_, 2, RC_FRAG, 2, false, true> : qgemm_stream_kernel<F, NI_, 1, RC_FRAG, 2, false, true>;
+    if (gw <= 4) return nullptr;
+    VQ_SG_TL(3) VQ_SG_TL(4) VQ_SG_TL(6) VQ_SG_TL(8)
+#undef VQ_SG_TL
+    return nullptr;
+}
+sg_fn sg_pick_tl4(int gw, bool pack);
+sg_fn sg_pick_tl8(int gw, bool pack);
 
 sg_fn sg_pick_q4(int gw, int am, bool pack, bool part, int senc, size_t* lds);
 sg_fn sg_pick_q5(int gw, int am, bool pack, bool part, int senc, size_t* lds);

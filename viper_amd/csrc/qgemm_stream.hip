@@ -154,4 +154,24 @@ int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, c
     return status_of(hipGetLastError());
 }
 
+int launch_sg_timeline(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int M,
+                       void* y, uint64_t* stamps, size_t stamp_bytes, int* workgroups, int* waves, hipStream_t st) {
+    SgLaunch l;
+    if (M < 2 || M > 16 || N >= (1 << 27) || !sg_launch(qtype, N, K, M, RC_FRAG, false, senc, l)) return VIPER_INVALID_ARGUMENT;
+    const int gw = (l.pg + SG_W - 1) / SG_W;
+    l.fn = qtype == VIPER_QTYPE_W8_G32 ? sg_pick_tl8(gw, M <= 8) : qtype == VIPER_QTYPE_Q4_G64 ? sg_pick_tl4(gw, M <= 8) : nullptr;
+    if (l.fn == nullptr) return VIPER_INVALID_ARGUMENT;
+    const unsigned nb = ((unsigned)N + (unsigned)l.rpw - 1) / (unsigned)l.rpw, gx = (nb + 7) / 8;
+    if (gx >= 1u << 20 || stamps == nullptr || stamp_bytes < (size_t)nb * SG_W * RC_TL_STAMPS * sizeof(uint64_t))
+        return VIPER_INVALID_ARGUMENT;
+    if (workgroups != nullptr) *workgroups = (int)nb;
+    if (waves != nullptr) *waves = SG_W;
+    const void* none = nullptr;
+    unsigned kk = (unsigned)(K / 32) | (unsigned)(l.pg - 1) << 20;
+    unsigned rg = (unsigned)l.rpw | gx << 12, ms = (unsigned)(M - 1) | (senc ? 16u : 0u);
+    void* args[] = {&xq, &xs, &w, &s, &y, &kk, &N, &rg, &ms, &none, &stamps, &none, &none, &none};
+    launch((const void*)l.fn, 8 * gx, 64 * SG_W, l.lds, st, args);
+    return status_of(hipGetLastError());
+}
+
 }  // namespace vq

@@ -6,5 +6,6 @@ namespace vq {
 sg_fn sg_pick_q4(int gw, int am, bool pack, bool part, int senc, size_t* lds) {
     return sg_pick<4>(gw, am, pack, part, senc, lds);
 }
+sg_fn sg_pick_tl4(int gw, bool pack) { return sg_pick_tl<4>(gw, pack); }
 
 }  // namespace vq

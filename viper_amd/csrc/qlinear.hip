@@ -649,6 +649,12 @@ extern "C" int viper_hip_qlinear_frag_timeline(int qtype, const void* w_packed, 
         return VIPER_INVALID_ARGUMENT;
     const size_t need = vq::frag_workspace_need(qtype, N, K, M);
     if (workspace != nullptr && (need == 0 || workspace_bytes < need)) return VIPER_INVALID_ARGUMENT;
+    // the kernel the production call runs, and only the calls its first kernel took
+    if (vq::frag_route(qtype, N, K, M, false, workspace != nullptr) == vq::R_SG) {
+        if (!vq::rc_timeline_ok(qtype, N, K, M, workspace != nullptr)) return VIPER_INVALID_ARGUMENT;
+        return vq::launch_sg_timeline(qtype, w_packed, w_scales, scale_enc, N, K, xfrag, xsfrag, M, y_bf16, stamps, stamp_bytes,
+                                      workgroups, waves_per_workgroup, (hipStream_t)stream);
+    }
     return vq::launch_rc_timeline(qtype, w_packed, w_scales, scale_enc, N, K, xfrag, xsfrag, M, y_bf16, stamps,
                                   stamp_bytes, workgroups, waves_per_workgroup, (unsigned*)workspace,
                                   (hipStream_t)stream);

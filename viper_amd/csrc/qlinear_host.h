@@ -169,6 +169,8 @@ bool rc_capped(int qtype, long rows_total, int K);
 int rc_rounds(int qtype, long rows_total, int K, int* rows);
 // A split launch's (row, part) pairs exceed two workgroups of 48 rows per CU.
 bool rc_split_capped(int qtype, int N, int K);
+// The calls the timeline entry point takes.
+bool rc_timeline_ok(int qtype, int N, int K, int M, bool split);
 int launch_rc_timeline(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq,
                        const void* xs, int M, void* y, uint64_t* stamps, size_t stamp_bytes, int* workgroups,
                        int* waves, unsigned* sc, hipStream_t st);
@@ -187,6 +189,8 @@ bool sg_takes(int qtype, int N, int K, int M, bool pair, int am);
 bool sg_over_mf(int qtype, int N, int K, int M, bool pair, int am);
 int sg_phases(int qtype, int K, int am);  // over K: what one workgroup's waves hold in registers
 bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair);
+int launch_sg_timeline(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int M,
+                       void* y, uint64_t* stamps, size_t stamp_bytes, int* workgroups, int* waves, hipStream_t st);
 int launch_sg(int qtype, const void* w, const void* s, int senc, int N, int K, const void* xq, const void* xs, int am,
               int M, void* y, const void* res, int32_t* part, const void* w1, const void* s1, void* y1, hipStream_t st);
 
