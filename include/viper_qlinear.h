@@ -92,7 +92,9 @@
  *
  * Alignment: w_packed, scales and x 16 bytes, xq 8 bytes, xs 4 bytes, y and
  * residual 2 bytes, partials 4 bytes.  Shapes: N, K, M > 0, K % G == 0,
- * M <= 16.
+ * M <= 16; 2..16 rows of a K of an odd number of groups, and one long row,
+ * up to 64 KiB of M staged int8 rows with their scales (K = 3520: 15 rows;
+ * INVALID_ARGUMENT past it).
  */
 #ifndef VIPER_QLINEAR_H
 #define VIPER_QLINEAR_H

@@ -74,7 +74,7 @@ def test_rmsnorm_qkv_equals_two_launches(torch_dev):
 @pytest.mark.parametrize("K,N", [(10240, 2560), (10752, 3072)])
 def test_swiglu_down_residual_equals_two_launches(torch_dev, K, N):
     # engine shapes: down (K=10240, N=2560; the reference's K=10752, N=3072 on
-    # the masked tiling) from silu(gate) * up, residual in place
+    # the streaming kernel) from silu(gate) * up, residual in place
     torch = torch_dev
     w = weights(torch, O.Q4_G64, N, K, 520)[0]
     rng = np.random.default_rng(521)
@@ -95,7 +95,7 @@ def test_swiglu_down_residual_equals_two_launches(torch_dev, K, N):
 # gate/up pair with the swiglu epilogue: equal, bit for bit, to the two GEMVs
 # of one viper_hip_qlinear_m1 launch followed by the standalone swiglu kernel;
 # the engine shape (rmsnorm prologue, K=2560, N=10240), the bf16 prologue,
-# every format, exact and masked tilings, ragged N, optional gate/up outputs.
+# every format, exact tilings and the streaming kernel, ragged N, optional gate/up outputs.
 @pytest.mark.parametrize("qtype,N,K,pro", [
     (O.Q4_G64, 10240, 2560, P.RMSNORM),
     (O.Q4_G64, 1000, 2560, P.BF16),
@@ -105,7 +105,7 @@ def test_swiglu_down_residual_equals_two_launches(torch_dev, K, N):
     (O.W8_G32, 777, 2560, P.BF16),
     (O.Q4_G64, 2560, 10240, P.BF16),
     (O.Q4_G64, 10752, 3072, P.RMSNORM),   # the reference engine's gate / up (6-slot tiling)
-    (O.Q5_G64, 1000, 10752, P.BF16),      # masked tiling
+    (O.Q5_G64, 1000, 10752, P.BF16),      # streaming kernel
 ])
 def test_gate_up_swiglu_equals_chain(torch_dev, qtype, N, K, pro):
     torch = torch_dev

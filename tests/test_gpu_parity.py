@@ -147,7 +147,7 @@ def test_multi_row_long_k(torch_dev, qtype, M, K):
 # M = 2..16 run on the i8 matrix cores when K is a multiple of two groups:
 # one load segment per wave (K <= 40 groups per 4 waves), the double-buffered
 # loop (long K), two 16-row tiles per wave (N >= 64 tiles per CU), partial
-# tiles, and K with an odd group count (the v_dot4 path).
+# tiles, and K with an odd group count (the streaming kernel).
 @pytest.mark.parametrize("qtype", FORMATS)
 @pytest.mark.parametrize("N,K,M,senc", [
     (16, 128, 2, O.SCALE_FP16),
@@ -156,7 +156,7 @@ def test_multi_row_long_k(torch_dev, qtype, M, K):
     (33, 6144, 7, O.SCALE_BF16),
     (16400, 256, 3, O.SCALE_FP16),
     (29, 192, 4, O.SCALE_FP16),
-    (300, 384, 9, O.SCALE_BF16),     # 6 groups (W8: 12): the pair-wise matrix-core kernel
+    (300, 384, 9, O.SCALE_BF16),     # 6 groups (W8: 12): gathered group pairs
     (70, 640, 12, O.SCALE_FP16),     # 10 groups (W8: 20)
     (1000, 3072, 16, O.SCALE_BF16),  # 12 quads: one per wave of 12 (W8: 24 quads, 3 parts of 8)
     (3000, 2816, 9, O.SCALE_FP16),   # 11 quads on 12 waves, the last one idle; 3000 rows: 48-row blocks
@@ -231,9 +231,9 @@ def test_k_split_random_shapes(torch_dev, qtype, N, K, M, senc):
 
 
 # Seeded random shapes through the bf16 entry, every dispatch path: 1..16
-# rows, K of 1..200 groups (odd group counts on the dot kernel, even ones on
-# the pair-swap matrix-core kernel, multiples of 4 on the row-contiguous one,
-# long K split or looped; M = 1 on exact, masked or general tilings), ragged
+# rows, K of 1..200 groups (odd group counts on the streaming kernel, even ones
+# there or on gathered pairs, multiples of 4 on the row-contiguous one, long K
+# split or looped; M = 1 on exact tilings or the streaming GEMV), ragged
 # N, both scale encodings, residual at random.  Group dots bit-exact through
 # the partials entry; the production entry's output equal to the partials
 # entry's bit for bit (the same arithmetic) and within the bar of the oracle.
@@ -493,8 +493,8 @@ def test_k_split_graph_replays(torch_dev):
 # heads): q 3072 -> 6144, k / v 3072 -> 1024, o 6144 -> 3072 (+ residual),
 # gate / up 3072 -> 10752, down 10752 -> 3072 (+ residual), full size, one
 # decode row and a 16-row verify, group dots bit-exact.  At M = 1 they run the
-# 6-slot exact tilings (K = 3072: 16 lanes per row, 6144: 32) and the masked
-# one (K = 10752: 336 chunks in 64 x 6 slots).
+# 6-slot exact tiling of K = 3072 (16 lanes per row) and the streaming GEMV
+# (K = 6144, unless a CU has 9..12 rows, and 10752: 336 chunks in 64 x 6 slots).
 @pytest.mark.parametrize("M", [1, 16])
 @pytest.mark.parametrize("N,K", [(6144, 3072), (1024, 3072), (3072, 6144), (10752, 3072), (3072, 10752)])
 def test_engine_shapes_full_size(torch_dev, N, K, M):
@@ -544,8 +544,8 @@ def test_m1_workgroup_choice(torch_dev, qtype, N, K):
 
 
 # Every format at the engine's K (ragged N, both scale encodings, outliers):
-# Q4 / Q5 / Q6 on the 6-slot and masked tilings, W8 on its own (K = 3072:
-# 32 lanes x 6, 6144: 64 x 6; 10752 on the general path).
+# Q4 / Q5 / Q6 on the 6-slot tiling of K = 3072, W8 on its own (32 lanes x 6),
+# the streaming GEMV else.
 @pytest.mark.parametrize("qtype", FORMATS)
 @pytest.mark.parametrize("N,K,senc", [(1000, 3072, O.SCALE_FP16), (777, 6144, O.SCALE_BF16),
                                       (1001, 10752, O.SCALE_FP16), (64, 10752, O.SCALE_BF16)])
@@ -700,7 +700,7 @@ def test_prequantized_m1(torch_dev, qtype, N, K):
     # M = 1 from int8 activations: the M = 1 kernel's prequantized prologue
     # (one octet per thread on 256 threads; Q4's two octets per thread on 320
     # and 640, a ragged last workgroup at N = 10010; the reference engine's K
-    # on the 6-slot tilings and the masked K = 10752 one; Q4 / Q5 at K = 3072
+    # on the 6-slot tilings and the streaming kernel; Q4 / Q5 at K = 3072
     # and N = 10752 / 11000 on the 44-row workgroup, ragged at 11000)
     torch = torch_dev
     G = O.group_size(qtype)
@@ -717,7 +717,7 @@ def test_prequantized_m1(torch_dev, qtype, N, K):
 
 # Two matrices of one shape on one activation in one launch (the reference's
 # fused2 for k/v and gate/up): M = 1 (fused quantize), M > 1 (matrix cores),
-# K with an odd group count (two v_dot4 launches).
+# K with an odd group count (the streaming kernel).
 @pytest.mark.parametrize("qtype", FORMATS)
 @pytest.mark.parametrize("N,K,M", [(300, 2560, 1), (5120, 2560, 1), (70, 2560, 16), (90, 2560, 6), (33, 192, 3)])
 @pytest.mark.parametrize("prequantized", [False, True])

@@ -500,7 +500,7 @@ static bool hm_takes(int M, int N, int K) {
 
 // Octets per thread of the split argmax.  Every workgroup's two atomics go to
 // the one or two cache lines that hold all rows' keys and counters and are
-// performed one after another there, ~15 ns each: with two octets per thread
+// performed one after another there, ~15 ns a workgroup: with two octets per thread
 // 166144 logits took 4.0 / 5.0 / 6.8 / 9.3 / 14.0 us for 1 / 2 / 4 / 8 / 16 rows,
 // with eight (a quarter of the workgroups) 4.1 / 4.1 / 4.5 / 5.0 / 6.0; 32000
 // logits 3.7 / 3.9 / 4.3 / 5.0 for 1 / 4 / 8 / 16 rows against 3.9 / 4.1 / 4.2 /

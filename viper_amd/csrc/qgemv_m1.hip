@@ -362,8 +362,8 @@ int launch_m1(int qtype, int senc, int K, int pro, const void* x, const void* xa
 
 int launch_m1_timeline(int qtype, int senc, int K, const void* x, const void* w, const void* s, void* y, int N,
                        uint64_t* stamps, size_t stamp_bytes, int* workgroups, int* waves, hipStream_t st) {
-    // rows that TS x CPL lanes and slots tile (5, 6 or 10 slots, or 336 chunks)
-    // and whose scales fill whole 16-byte words
+    // rows of 5 or 10 (6) slots of 16, 32 or 64 lanes, or of 336 chunks, whose
+    // scales fill whole 16-byte words, on the kernel that the call runs
     const int ck = qtype == VIPER_QTYPE_W8_G32 ? 16 : 32, group = qtype == VIPER_QTYPE_W8_G32 ? 32 : 64;
     const int cpr = K / ck;
     if ((cpr != 80 && cpr != 160 && cpr != 320 && cpr != 640 && cpr != 96 && cpr != 192 && cpr != 384 && cpr != 336) ||

@@ -430,11 +430,13 @@ qgemv_stream_kernel(const void* x, const uint8_t* w0, const uint16_t* s0, uint16
 
 // Launch shapes: (team size, chunk slots per lane, rows per team of a unit).
 // The team is the narrowest that covers the row in two slots up to 64 chunks
-// (K = 2048; W8 1024; one slot up to 8 chunks), then 64 lanes with as many slots as the row needs.
+// (K = 2048; W8 1024; one slot up to 8 chunks), then 64 lanes with as many slots as the row needs.  The
+// timeline only for the rows its entry point takes that no tiling always
+// covers: 160 to 640 chunks.
 template <int F, int SENC, int MODE, int PRO>
 m1_fn st_kernel_v(int ts, int cpl, int r) {
 #define VQ_ST(TS_, CPL_, R_) \
-    if constexpr (CPL_ <= ST_MAX<F>)  \
+    if constexpr (CPL_ <= ST_MAX<F> && (MODE != M1_TL || (CPL_ == 3 && F != 8) || CPL_ == 5 || CPL_ == 6 || CPL_ == ST_MAX<F>)) \
         if (ts == TS_ && cpl == CPL_ && r == R_) return qgemv_stream_kernel<F, TS_, CPL_, R_, SENC, MODE, PRO>;
     VQ_ST(8, 1, 1) VQ_ST(8, 2, 1) VQ_ST(16, 2, 1) VQ_ST(32, 2, 1) VQ_ST(64, 2, 1) VQ_ST(64, 2, 2) VQ_ST(64, 3, 1) VQ_ST(64, 4, 1)
     VQ_ST(64, 5, 1) VQ_ST(64, 6, 1) VQ_ST(64, 7, 1) VQ_ST(64, 8, 1) VQ_ST(64, 9, 1) VQ_ST(64, 10, 1)

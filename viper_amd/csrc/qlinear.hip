@@ -15,8 +15,8 @@
 // v_dot4 on offset codes for Q5/Q6/W8) and the fp32 combine is reduced with
 // DPP in a fixed order (deterministic).
 //
-// M = 2..16 (qgemm_rc.h, qgemm_stream.h): few rows are quantized by every
-// workgroup, more are quantized once into a caller workspace in the
+// M = 2..16 (qgemm_rc.h, qgemm_stream.h, qgemm_mfma.hip; which one is the Route
+// of a call below): few rows are quantized by every workgroup, more are quantized once into a caller workspace in the
 // matrix-core fragment order or supplied by the caller, and every weight byte
 // is read once for all M rows.
 //
@@ -397,7 +397,8 @@ static Route frag_route(int qtype, int N, int K, int M, bool pair, bool ws) {
 }
 
 // The rows' limit of a call that neither the M = 1 kernels nor the
-// row-contiguous kernel take: one row, or K of an odd number of groups.
+// row-contiguous kernel take: one row, or K of an odd number of groups.  (The
+// entry points' limit: their callers' refusals stay, whichever kernel runs.)
 static bool rows_refused(int qtype, int M, int K) {
     return (M < 2 || (K / group_of(qtype)) % 2 != 0) && lds_pre(qtype, M, K) > (size_t)LDS_MAX;
 }
@@ -473,10 +474,10 @@ static int prequant_common(int qtype, const void* w, const void* s, int senc, in
 }
 
 // 2..16 int8 rows already in the matrix-core fragment order (a producer's
-// fragment output): one launch of the row-contiguous matrix-core kernel.  Long
-// K splits over workgroups when a workspace of frag_workspace_need bytes is
-// given (no launch before it: the split keeps its own counters), else runs
-// the segment loop.
+// fragment output): one launch of the row-contiguous matrix-core kernel, or of
+// the streaming one where the rows exceed one round of it.  Long K splits over
+// workgroups when a workspace of frag_workspace_need bytes is given (no launch
+// before it: the split keeps its own counters), else runs the segment loop.
 static int prequant_frag(int qtype, const void* w, const void* s, int senc, int group, int N, int K,
                          const void* xf, const void* xsf, int M, void* y, const void* res, void* wsp,
                          size_t wsp_bytes, void* stream, Second b = Second()) {

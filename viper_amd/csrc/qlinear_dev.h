@@ -13,7 +13,6 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int NT = 256;            // threads per workgroup (generic kernels)
-constexpr int CPL = 8;             // chunk slots per lane per row segment (generic kernel)
 constexpr int LDS_MAX = 65536;     // dynamic LDS budget per workgroup
 
 template <int F> struct Fmt;
