@@ -77,3 +77,12 @@ def test_route_padding(qtype, rows, N, K, M, matrices, want):
     (W8, BF16, 256, 13248, 12, STREAM), (Q4, BF16, 24576, 384, 8, PAIRS), (Q4, BF16, 2560, 3456, 8, STREAM_BF16)])
 def test_route_pairs(qtype, rows, N, K, M, want):
     assert route(qtype, rows, N, K, M) == want
+
+
+# Two bf16 rows over several rounds of the row-contiguous kernel: the kernel that pads fewest; a long K of a pair stays in
+# one launch.
+@pytest.mark.parametrize("qtype,N,K,matrices,want", [
+    (Q4, 17366, 1536, 1, ROWS), (Q4, 20480, 2048, 1, ROWS), (Q4, 24320, 2048, 1, RC_BF16), (Q4, 12800, 1792, 1, ROWS),
+    (Q5, 14000, 2048, 1, STREAM_BF16), (Q4, 20000, 2048, 2, RC_BF16), (Q5, 20000, 2048, 2, RC), (Q6, 25600, 1536, 1, ROWS), (W8, 26645, 5504, 2, RC_BF16), (Q4, 20736, 256, 1, RC_BF16)])
+def test_route_two_rows_padding(qtype, N, K, matrices, want):
+    assert route(qtype, BF16, N, K, 2, matrices) == want

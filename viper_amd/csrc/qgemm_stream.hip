@@ -70,8 +70,8 @@ bool sg_bf16_ok(int qtype, int N, int K, int M, bool pair) {
 // 3328 9.7 / 10.5, 16 int8 rows of K = 4608 14.4 / 16.3; of K = 4096, whole steps,
 // 13.9 / 11.9; fragments of K = 3328 10.4 / 10.0, 7 int8 rows of a pair of K =
 // 3584 20.8 / 18.6; Q6, N = 10000, 4 bf16 rows of K = 3328 12.1 / 10.7).
-// Two bf16 rows also leave the other kernels of that family for one that pads
-// fewer rows (Q5, K = 2048, N = 14000 11.3 / 8.3; Q4 8.1 / 7.5).
+// Two bf16 rows, up to 64 per CU, also leave the other kernels of that family
+// for one that pads fewer rows (Q5, K = 2048, N = 14000 11.3 / 8.3).
 bool sg_takes(int qtype, int N, int K, int M, bool pair, int am) {
     if (!rc_ok(qtype, K)) return true;
     const long total = sg_rows(N, pair);
@@ -81,7 +81,7 @@ bool sg_takes(int qtype, int N, int K, int M, bool pair, int am) {
     const int rounds = rc_rounds(qtype, total, K, &rows);
     const long per_cu = (total + device_cus() - 1) / device_cus();
     if (!rc_capped(qtype, total, K))
-        return am == RC_BF16 && M == 2 && !pair && rounds > 1 && (per_cu + 15) / 16 * 16 < (long)rounds * rows;
+        return am == RC_BF16 && M == 2 && !pair && rounds > 1 && per_cu <= 64 && (per_cu + 15) / 16 * 16 < (long)rounds * rows;
     const int gw = (K / group_of(qtype) + SG_W - 1) / SG_W;
     const bool even = rows > 16 && (per_cu + 15) / 16 * 16 == (long)rounds * rows && gw % 4 != 0;
     return !(even && !pair && ((am == RC_NAT && M > 8 && qtype != VIPER_QTYPE_Q6_G64) ||

@@ -280,7 +280,8 @@ static int validate_second(const Second& b, int qtype, int senc, int group, int 
 // least while one round of 40-row workgroups holds them here, 33..40 rows per
 // CU (N = 10240: Q4 K = 2112 5.6 / 6.5, K = 4608 8.1 / 9.7; Q6 K = 2112 6.9 / 7.7;
 // W8 K = 1760 5.4 / 6.2; N = 8192 the other way; Q4, K = 4096, N = 11005, two
-// rounds, 12.3 / 8.2), short rows of W8, which decodes cheapest, from there on
+// rounds, 12.3 / 8.2; up to 36 groups of Q4 also those two rounds, 49..80 rows:
+// N = 14080, K = 1280 6.8 / 7.05, K = 2304 7.8 / 8.6), short rows of W8, which decodes cheapest, from there on
 // (N = 16384, K = 704 4.8 / 5.8, K = 1056 5.9 / 6.7), and few long ones of it,
 // whose tiles take the most steps (K = 3520, N = 2560 6.3 / 6.5; K = 4096, N =
 // 4256 6.7 / 8.9, N = 6144 equal).
@@ -288,8 +289,9 @@ static bool dot_rows(int qtype, int N, int K, int M, bool one, bool takes) {
     if (!m1_rows_ok(qtype, K, M)) return false;
     if (m1_rows_exact(qtype, K, M) || !one) return true;
     if (M > 2 || !takes) return false;
-    const bool w8 = qtype == VIPER_QTYPE_W8_G32;
+    const bool w8 = qtype == VIPER_QTYPE_W8_G32, q4 = qtype == VIPER_QTYPE_Q4_G64;
     const long per_cu = (N + (long)device_cus() - 1) / device_cus();
+    if (q4 && K <= 2304 && per_cu > 48 && per_cu <= 80) return true;
     return (per_cu > 32 && (per_cu <= 40 || (w8 && K <= 1152))) || (w8 && K > 96 * 32 && per_cu <= 20);
 }
 
@@ -321,7 +323,17 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     const bool one = sg_bf16_ok(qtype, N, K, M, pair);
     const bool takes = sg_takes(qtype, N, K, M, pair, one ? RC_BF16 : RC_FRAG);
     const bool dot = !pair && dot_rows(qtype, N, K, M, one, takes);
-    if (M == 2 && dot) return R_ROWS;
+    int wg_rows;
+    const int rounds = rc_k ? rc_rounds(qtype, pair ? 2L * N : N, K, &wg_rows) : 0;
+    // (two rows past 64 per CU, several rounds of the row-contiguous kernel of up
+    // to 48 rows: the dots where rounds of their 40 pad fewer; Q4, K = 1536, N =
+    // 17366 7.4 us against 9.9 on the streaming kernel, K = 2048, N = 20480 8.4 /
+    // 9.7; Q6, K = 1536, N = 25600 12.7 against 15.3 on the row-contiguous one; Q4,
+    // K = 2048, N = 24320 10.1 / 9.6)
+    const long per_cu = (N + (long)device_cus() - 1) / device_cus();
+    const bool dots_pad = !pair && !takes && rounds > 1 && per_cu > 64 && (per_cu + 39) / 40 * 40 < (long)rounds * wg_rows &&
+                          m1_rows_ok(qtype, K, M);
+    if (M == 2 && (dot || dots_pad)) return R_ROWS;
     // With the rows staged two octets per thread (64-groups), the row-contiguous
     // kernel's one-launch path also wins for Q4 at 3-4 rows (5.45 / 5.74 against
     // 5.6 / 5.9 us on the dot kernel) and 9-10 rows (6.76 / 7.00 against 7.27 us
@@ -331,14 +343,13 @@ static Route linear_route(int qtype, int N, int K, int M, bool pair, bool part) 
     // workgroups quantizes the rows again: where the streaming kernel would
     // take two launches, up to 12 rows times rounds (Q4, K = 7168: 3 rows, N =
     // 10240 15.6 against 16.5 us, 5 rows, N = 8192 / 10240 13.4 / 18.7 against
-    // 13.5 / 16.5); a pair's two rows up to two rounds (Q5, K = 2048, N = 24576
-    // 23.2 against 21.7 us in two launches).
+    // 13.5 / 16.5); a pair's two rows of Q5 and Q6 and a K of one phase up to two
+    // rounds (Q5, K = 2048, N = 20000 22.1 against 20.7 us in two launches; Q4 16.2 /
+    // 17.5; Q5, K = 5504 45.7 / 61.4).
     const bool q4 = qtype == VIPER_QTYPE_Q4_G64;
     const int bf_max = q4 && !pair ? 10 : 8;
-    int wg_rows;
-    const int rounds = rc_k ? rc_rounds(qtype, pair ? 2L * N : N, K, &wg_rows) : 0;
     const bool rc_bf16 = rc_k && M <= bf_max && rc_bf16_ok(qtype, N, K, M, pair) && (!takes || (!one && M * rounds <= 12)) &&
-                         !(pair && M == 2 && rounds > 2);
+                         !(pair && M == 2 && rounds > 2 && !q4 && qtype != VIPER_QTYPE_W8_G32 && sg_phases(qtype, K, RC_FRAG) == 1);
     // Long K splits over workgroups in the two-launch path (down shape
     // K = 10240, 4 rows 9.5 us against 10.3 us without the split), unless one
     // launch serves a K of one phase (Q4, 6 rows, K = 6144, N = 3072 6.8 us
