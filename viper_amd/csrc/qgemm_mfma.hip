@@ -1,6 +1,9 @@
-// M = 2..16: quantized skinny GEMM on the i8 matrix cores of gfx950, for K a
-// multiple of two groups that the row-contiguous kernels (qgemm_rc.h, K a
-// multiple of four groups) do not take.
+// M = 2..16: quantized skinny GEMM on the i8 matrix cores of gfx950, for K of
+// an even number of groups that is no multiple of four (qgemm_rc.h takes
+// those), where it is faster than the streaming kernel (qgemm_stream.h; the
+// rule and both sides' figures at sg_over_mf).  Bound by the latency of its one
+// or few load segments: Q4, 16 rows, K = 384, N = 24576 5.7 us from int8 rows
+// (0.9 TB/s of weights), K = 3712, N = 24000 18.5 us (2.6 TB/s).
 //
 // Semantics are those of the reference's multi-row path
 // (kernels/ops/linear_multim.cu:64-130): per group, the int32 dot of the
@@ -355,18 +358,18 @@ template <int F, bool ONE, bool XNAT, bool PART>
 static mf_fn mf_kernel_v(int t, int w) {
 #define VQ_MF(T_, W_) \
     if (t == T_ && w == W_) return qgemm_mfma_kernel<F, T_, W_, ONE, XNAT, PART>;
-    VQ_MF(1, 4) VQ_MF(1, 8) VQ_MF(2, 4) VQ_MF(2, 8)
+    if constexpr (ONE) { VQ_MF(1, 4) VQ_MF(2, 4) }  // (four waves: always one segment, mf_shape)
+    VQ_MF(1, 8) VQ_MF(2, 8)
 #undef VQ_MF
     return nullptr;
 }
-template <int F, bool PART>
-static mf_fn mf_kernel_p(int t, int w, bool one, bool xnat) {
-    if (one) return xnat ? mf_kernel_v<F, true, true, PART>(t, w) : mf_kernel_v<F, true, false, PART>(t, w);
-    return xnat ? mf_kernel_v<F, false, true, PART>(t, w) : mf_kernel_v<F, false, false, PART>(t, w);
-}
+// (the group dots are asked for from bf16 rows only, which arrive as fragments)
 template <int F>
 static mf_fn mf_kernel(int t, int w, bool one, bool xnat, bool part) {
-    return part ? mf_kernel_p<F, true>(t, w, one, xnat) : mf_kernel_p<F, false>(t, w, one, xnat);
+    if (part && xnat) return nullptr;
+    if (part) return one ? mf_kernel_v<F, true, false, true>(t, w) : mf_kernel_v<F, false, false, true>(t, w);
+    if (one) return xnat ? mf_kernel_v<F, true, true, false>(t, w) : mf_kernel_v<F, true, false, false>(t, w);
+    return xnat ? mf_kernel_v<F, false, true, false>(t, w) : mf_kernel_v<F, false, false, false>(t, w);
 }
 
 // Tiles of 16 rows per workgroup and waves per workgroup: two tiles per wave

@@ -450,13 +450,12 @@ static int qlinear_common(int qtype, const void* w, const void* s, int senc, int
     // the workspace's start, then the records of part sums)
     uint64_t* sp = route == R_SPLIT ? (uint64_t*)((uint8_t*)wsp + lay.sp) : nullptr;
     unsigned* sc = route == R_SPLIT ? (unsigned*)wsp : nullptr;
-    const bool nat = route == R_MF && !mf_frag_ok(qtype, N, K);
-    rc = launch_quantize(group, x, M, K, xq, xs, !nat, st);
+    rc = launch_quantize(group, x, M, K, xq, xs, true, st);
     if (rc != VIPER_OK) return rc;
     if (route == R_SG)
         return launch_sg(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st);
     if (route == R_MF)
-        return launch_mf(qtype, w, s, senc, N, K, xq, xs, nat, M, y, res, part, b.w, b.s, b.y, st);
+        return launch_mf(qtype, w, s, senc, N, K, xq, xs, false, M, y, res, part, b.w, b.s, b.y, st);
     return launch_rc(qtype, w, s, senc, N, K, xq, xs, RC_FRAG, M, y, res, part, b.w, b.s, b.y, st, sp, sc);
 }
 
